@@ -36,6 +36,16 @@ constexpr uint32_t PREFILL_MIN_T = 16;
 // by ~1e-5 * e^-LOGN * max|v - out| even when all of them push the same way.
 constexpr float PREFILL_TAU_MIN = 7.0f;
 constexpr float PREFILL_TAU_LOGN = 2.0f;
+// The prefill split's cost model (prefill_split), in the time of one 16-key tile
+// of a workgroup (1.3 us at head_dim 256, 2.6 at 512): a workgroup's fixed cost,
+// the merge launch, a partial slot's write and read; the fewest tiles worth a
+// share; and the most partial slots of a call (132 KiB each at head_dim 512).
+constexpr float PREFILL_WG_TILES_256 = 18.0f;
+constexpr float PREFILL_WG_TILES_512 = 11.0f;
+constexpr float PREFILL_MERGE_TILES = 3.0f;
+constexpr float PREFILL_SLOT_TILES = 0.02f;
+constexpr uint32_t PREFILL_MIN_SHARE = 2;
+constexpr uint32_t PREFILL_MAX_SLOTS = 1024;
 // Largest split-K count the LSE combine kernel takes (its LDS weight table).
 constexpr uint32_t MAX_SPLITS = 1024;
 // Split counts merged by the one-block-per-head combine kernel (combine_rows).
@@ -53,8 +63,12 @@ constexpr uint32_t BATCH_MAX_KEYS = SHORT_KEYS * MAX_SPLITS;
 // their own.
 thread_local std::string g_create_error;
 
-// Bytes of the static scratch array a call that allocates nothing may use.
+// Bytes of the static scratch array a call that allocates nothing may use, and
+// of the part behind them that only a prefill's split partials take (256
+// workgroups of head_dim 512): a call that fits the former always has room for
+// enough of them.
 constexpr size_t NOALLOC_SCRATCH_BYTES = G4A_NOALLOC_SCRATCH_BYTES;
+constexpr size_t NOALLOC_PARTIAL_BYTES = size_t(34) << 20;
 
 // Tags each K/V pre-split's V range flag (G4aSplitParams::epoch). Process-wide,
 // so no two pre-splits of any context share a tag.
@@ -73,7 +87,7 @@ uint32_t next_split_epoch() {
 // array, at its own address, from the first context on it until the process
 // ends. In host code `scratch` names a host-side stand-in, not device memory:
 // kernels get the device address from scratch_setup, never the name itself.
-static __device__ __align__(256) unsigned char scratch[G4A_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[G4A_NOALLOC_SCRATCH_BYTES + NOALLOC_PARTIAL_BYTES];
 
 // The graphs captured on a context, shared by the context and each of its
 // graphs. A graph replays with the workspace it was captured with, so while
@@ -109,6 +123,7 @@ struct g4a_ctx {
     uint32_t short_ds = 4;     // g4a_options::short_max_wgs: most workgroups per short split
     hipFunction_t generic = nullptr;
     hipFunction_t prefill[2] = {nullptr, nullptr};                          // [dh512]
+    hipFunction_t prefill_whole = nullptr;  // head_dim 256, no query block split
     hipFunction_t split_kv = nullptr;  // K/V pre-split for the head_dim 256 prefill
     hipFunction_t norm_rope = nullptr;        // the attention producer (RMSNorm + RoPE + KV write)
     hipFunction_t norm_rope_short = nullptr;  // the same with its loads issued together (<= 1 workgroup per CU)
@@ -159,7 +174,7 @@ struct g4a_ctx {
     size_t prev_workspace_bytes = 0;  // the size of the buffer the last growth replaced
     int query_depth = 0;              // > 0 inside a query entry point (g4a_attention_plan)
     void* scratch = nullptr;  // this device's static scratch array (the allocation-free entry point)
-    hipFunction_t prefill_merge = nullptr;  // merge of the split hd512 prefill blocks
+    hipFunction_t prefill_merge[2] = {nullptr, nullptr};  // [dh512] merge of split prefill blocks
     float* dummy = nullptr;  // 4 KiB of zeros: the load target of idle decode tiles
     uint32_t* pos_dev = nullptr;  // device copies of non-contiguous positions
     size_t pos_dev_cap = 0;       // in u32
@@ -273,32 +288,137 @@ int ensure_workspace(g4a_ctx* ctx, size_t bytes) {
     return G4A_OK;
 }
 
-// Query blocks of the head_dim 512 prefill that run as two workgroups, one per
-// half of their key tiles: the trailing blocks (causal masks give later queries
-// more keys) whose tile count exceeds the average over all blocks. Mirrors the
-// kernel's tile range of a block of 8 queries (prefill_dsplit).
-uint32_t prefill_split_blocks(const g4a_attn_args* a, uint32_t q_pos0, uint32_t k_pos0) {
-    const uint32_t NB = (a->T + 7) / 8;
-    if (NB == 0) return 0;
-    auto key_hi = [&](int64_t i) -> int64_t {
-        const int64_t lim = (int64_t)q_pos0 + i - (int64_t)k_pos0 + 1;
-        return lim <= 0 ? 0 : std::min<int64_t>(lim, a->S);
+// 16-key tiles of each block of 8 queries of a prefill call, as the kernels
+// count them (prefill_pair, prefill_dsplit).
+struct PrefillTiles {
+    const g4a_attn_args* a;
+    uint32_t q_pos0, k_pos0;
+    uint32_t operator()(uint32_t b) const {
+        const int64_t off = (int64_t)q_pos0 - (int64_t)k_pos0 + 1;
+        const int64_t last = std::min<int64_t>(8 * int64_t(b) + 7, int64_t(a->T) - 1);
+        const int64_t hi = std::min<int64_t>(std::max<int64_t>(off + last, 0), a->S);
+        const int64_t lo = a->sliding_window == 0
+                               ? 0
+                               : std::min<int64_t>(std::max<int64_t>(off + 8 * int64_t(b) - a->sliding_window, 0), a->S);
+        return hi > lo ? uint32_t((hi - (lo & ~int64_t(15)) + 15) / 16) : 0;
+    }
+};
+
+// How a prefill's query blocks are split over workgroups (G4aPrefillParams::cls_nb).
+struct PrefillSplit {
+    uint32_t ncls = 0, nb[G4A_PF_CLASSES] = {}, ns[G4A_PF_CLASSES] = {};
+    uint32_t blocks = 0;  // workgroups per kv head
+    uint32_t split = 0;   // query blocks of more than one workgroup
+    uint32_t slots = 0;   // their workgroups: partial slots per kv head
+};
+
+// A query block's workgroups when its heaviest block has `most`: shares of at
+// most `tpi` tiles, in steps that keep the counts to G4A_PF_CLASSES.
+uint32_t prefill_shares(uint32_t nt, uint32_t tpi, uint32_t most) {
+    const uint32_t step = (most + G4A_PF_CLASSES - 2) / (G4A_PF_CLASSES - 1);
+    const uint32_t n = (nt + tpi - 1) / tpi;
+    return n <= 1 ? 1 : std::min(most, (n + step - 1) / step * step);
+}
+
+// Splits every block at `tpi` tiles a share, `most` shares at most.
+PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, uint32_t tpi, uint32_t most) {
+    PrefillSplit sp;
+    // from the first block on, the share count never decreases (a window's tile
+    // counts move up and down by one with its alignment)
+    uint32_t nb[G4A_PF_CLASSES] = {}, ns[G4A_PF_CLASSES] = {1}, n = 0;
+    for (uint32_t b = 0; b < NB; ++b) {
+        const uint32_t s = prefill_shares(tiles(b), tpi, most);
+        if (s > ns[n]) {
+            if (nb[n]) ++n;
+            ns[n] = s;
+        }
+        ++nb[n];
+    }
+    for (int c = int(n); c >= 0; --c) {
+        sp.nb[sp.ncls] = nb[c];
+        sp.ns[sp.ncls++] = ns[c];
+        sp.blocks += nb[c] * ns[c];
+        if (ns[c] > 1) sp.split += nb[c], sp.slots += nb[c] * ns[c];
+    }
+    return sp;
+}
+
+// Chooses the split by the time the launch would take. A prefill workgroup fills
+// a CU (LDS) and costs its tiles plus a fixed part (loading q, the exact
+// rescoring of its candidates); the workgroups start in order, the heaviest
+// blocks' first, each on the CU that frees first, which is played through here
+// at a scale of PF_SIM_CUS; a split block adds the traffic of its partials and a
+// merge launch. Tried: share counts of the heaviest block spaced by about a
+// quarter, the one that just fills the CUs, and halving the blocks above the
+// mean, on up to 64 sampled blocks.
+// Against a sweep of fixed counts the choice is within 5 % of the best over T =
+// 16 .. 2048 and up to 16000 earlier keys (us, one workgroup a block -> chosen):
+// hd512 T = 173 after 6001 keys 1048 -> 168, 16 after 16000 2639 -> 128, T = 2048
+// 385 -> 317 (363 with the later blocks halved), 231 74 -> 44; hd256 window 512,
+// T = 2048 unchanged, 512 79 -> 46, 120 after 3000 83 -> 43.
+constexpr int PF_SIM_CUS = 32;
+
+PrefillSplit prefill_split(const PrefillTiles& tiles, uint32_t NB, uint32_t Hkv, uint64_t cus, bool d512,
+                           uint32_t max_slots) {
+    const float fixed = d512 ? PREFILL_WG_TILES_512 : PREFILL_WG_TILES_256;
+    const uint32_t n = std::min<uint32_t>(NB, 64);
+    uint32_t nt[64], top = std::max(tiles(NB - 1), 1u);
+    for (uint32_t i = 0; i < n; ++i) {
+        nt[i] = tiles(uint32_t((uint64_t(i) * 2 + 1) * NB / (2 * n)));
+        top = std::max(top, nt[i]);
+    }
+    const double each = double(NB) * Hkv / n;  // blocks a sample stands for
+    auto rounds = [&](uint32_t tpi, uint32_t most) {
+        float busy[PF_SIM_CUS] = {};
+        const float w = float(each * PF_SIM_CUS / double(cus));
+        float due = 0.0f;
+        for (uint32_t i = n; i-- > 0;) {
+            const uint32_t s = prefill_shares(nt[i], tpi, most);
+            const float cost = float(nt[i]) / float(s) + fixed;
+            for (due += float(s) * w; due >= 1.0f; due -= 1.0f) *std::min_element(busy, busy + PF_SIM_CUS) += cost;
+        }
+        return *std::max_element(busy, busy + PF_SIM_CUS);
     };
-    auto key_lo = [&](int64_t i) -> int64_t {
-        if (a->sliding_window == 0) return 0;
-        const int64_t lo = (int64_t)q_pos0 + i - (int64_t)k_pos0 - (int64_t)a->sliding_window + 1;
-        return lo <= 0 ? 0 : std::min<int64_t>(lo, a->S);
+    float best = 3.0e38f;
+    uint32_t best_tpi = top, best_most = 1;
+    auto consider = [&](uint32_t tpi, uint32_t most) {
+        if (most > 1 && tpi < PREFILL_MIN_SHARE) return;
+        double items = 0, slots = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            const uint32_t s = prefill_shares(nt[i], tpi, most);
+            items += s;
+            if (s > 1) slots += s;
+        }
+        items *= each, slots *= each;
+        // (many rounds more than the unsplit launch's gain nothing)
+        if (slots > max_slots || (most > 1 && items > 4.0 * double(cus) && items > 1.5 * each * n)) return;
+        float est = std::max(float(tpi), float(top) / float(most)) + fixed;
+        if (items > double(cus)) est = std::max(est, rounds(tpi, most));
+        if (slots > 0) est += PREFILL_MERGE_TILES + float(slots) * PREFILL_SLOT_TILES;
+        if (est < best) best = est, best_tpi = tpi, best_most = most;
     };
-    auto tiles = [&](uint32_t b) -> int64_t {  // 16-key tiles of query block b
-        const int64_t lo = key_lo(8 * int64_t(b)), hi = key_hi(std::min<int64_t>(8 * int64_t(b) + 7, a->T - 1));
-        const int64_t base = lo & ~int64_t(15);
-        return hi > lo ? (hi - base + 15) / 16 : 0;
-    };
-    int64_t total = 0;
+    auto even = [&](uint32_t most) { consider((top + most - 1) / most, most); };
+    for (uint32_t most = 1; most <= G4A_PF_MAX_SHARES; most = most < 4 ? most + 1 : most + most / 4) even(most);
+    const uint64_t fill = cus / (uint64_t(NB) * Hkv);
+    if (fill > 1) even(uint32_t(std::min<uint64_t>(fill, G4A_PF_MAX_SHARES)));
+    uint64_t sum = 0;
+    for (uint32_t i = 0; i < n; ++i) sum += nt[i];
+    consider(uint32_t(sum / n) + 1, 2);  // only the blocks above the mean, halved
+    const PrefillSplit sp = prefill_split_at(tiles, NB, best_tpi, best_most);
+    // (the sampled tile counts can miss the limit)
+    return uint64_t(sp.slots) * Hkv <= max_slots ? sp : prefill_split_at(tiles, NB, top, 1);
+}
+
+// Bytes of partials g4a_attention_noalloc counts against its static array, which
+// sets what it refuses: at head_dim 512, two 132 KiB halves for each trailing
+// block of more tiles than the average.
+size_t noalloc_partial_bytes(const PrefillTiles& tiles, bool d512) {
+    if (!d512) return 0;
+    const uint32_t NB = (tiles.a->T + 7) / 8;
+    uint64_t total = 0, nbig = 0;
     for (uint32_t b = 0; b < NB; ++b) total += tiles(b);
-    uint32_t nbig = 0;
-    while (nbig < NB && tiles(NB - 1 - nbig) * int64_t(NB) > total) ++nbig;
-    return nbig;
+    while (nbig < NB && uint64_t(tiles(NB - 1 - uint32_t(nbig))) * NB > total) ++nbig;
+    return size_t(nbig) * tiles.a->Hkv * 2 * 8 * (4 * 16 * 64 + 32) * sizeof(float);
 }
 
 // Stages up to two host position arrays into device memory (stream-ordered).
@@ -600,9 +720,11 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
     if (int rc = get_fn(ctx, &ctx->combine[0], "g4a_combine_d256")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->combine[1], "g4a_combine_d512")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->generic, "g4a_generic_attention")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->prefill[0], "g4a_prefill2_d256")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->prefill[0], "g4a_prefill2_split_d256")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->prefill_whole, "g4a_prefill2_d256")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->prefill[1], "g4a_prefill2_d512")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->prefill_merge, "g4a_prefill_merge_d512")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->prefill_merge[0], "g4a_prefill_merge_d256")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->prefill_merge[1], "g4a_prefill_merge_d512")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->split_kv, "g4a_split_kv")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->norm_rope, "g4a_norm_rope")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->norm_rope_short, "g4a_norm_rope_short")) return bail(rc);
@@ -863,20 +985,29 @@ int attention_run(g4a_ctx* ctx, const g4a_attn_args* a, const Analysis& an, bool
         // head_dim 256: two waves per 16-row block take the even / odd key tiles;
         // 512: two waves per 16-row block split the head dim
         const bool d512 = a->Dh == 512;
+        PrefillSplit split;
         {
             // keys [k_start, k_end) widened to multiples of 16 (the kernel's tile grid);
             // workspace: the V range flag (first 256 bytes), then the K and V splits,
-            // the K rows' scale factors, then (head_dim 512) the partials of the split
-            // query blocks
+            // the K rows' scale factors, then the partials of the split query blocks
             const uint32_t k0 = pl.k_start & ~15u, nkeys = ((pl.k_end + 15u) & ~15u) - k0;
             const size_t half = size_t(nkeys) * a->Hkv * a->Dh * sizeof(float);
             const size_t kscale_bytes = size_t(a->Hkv) * (nkeys / 16) * sizeof(float);
-            if (d512) pp.nbig = prefill_split_blocks(a, pp.q_pos0, pp.k_pos0);
-            // a split block's partial: 8 waves x (O of 16 rows x 256 dims, then l and m of the rows)
-            const size_t part_bytes = size_t(pp.nbig) * a->Hkv * 2 * 8 * (4 * 16 * 64 + 32) * sizeof(float);
             const size_t part_off = (256 + 2 * half + kscale_bytes + 255) & ~size_t(255);
+            // a slot: 8 waves at head_dim 512, 4 at 256, of 16 rows x 256 columns, l and m
+            const size_t slot_bytes = size_t(d512 ? 8 : 4) * (16 * 256 + 2 * 16) * sizeof(float);
+            // the static array bounds the partials of every call whose splits fit it, so that
+            // g4a_attention_noalloc runs the same split as g4a_attention
+            const size_t room = part_off <= NOALLOC_SCRATCH_BYTES
+                                    ? NOALLOC_SCRATCH_BYTES + NOALLOC_PARTIAL_BYTES - part_off
+                                    : SIZE_MAX;
+            const PrefillTiles tiles{a, pp.q_pos0, pp.k_pos0};
+            split = prefill_split(tiles, (a->T + 7) / 8, a->Hkv, uint64_t(std::max(ctx->cu_count, 1)), d512,
+                                  uint32_t(std::min<size_t>(room / slot_bytes, PREFILL_MAX_SLOTS)));
+            const size_t need = part_off + (noalloc ? noalloc_partial_bytes(tiles, d512)
+                                                    : split.slots * a->Hkv * slot_bytes);
             void* wsp = nullptr;
-            if (int rc = call_workspace(ctx, part_off + part_bytes, noalloc, &wsp)) return rc;
+            if (int rc = call_workspace(ctx, need, noalloc, &wsp)) return rc;
             char* const ws = static_cast<char*>(wsp);
             G4aSplitParams sp{};
             sp.k = a->k;
@@ -909,12 +1040,16 @@ int attention_run(g4a_ctx* ctx, const g4a_attn_args* a, const Analysis& an, bool
             pp.epoch = sp.epoch;
             pp.part = reinterpret_cast<float*>(ws + part_off);
         }
-        if (int rc = launch(ctx, ctx->prefill[d512 ? 1 : 0], dim3((a->T + 7) / 8 + pp.nbig, a->Hkv, 1),
-                            dim3(512, 1, 1), pp, "prefill", true))
+        pp.part_slots = split.slots;
+        pp.ncls = split.ncls;
+        memcpy(pp.cls_nb, split.nb, sizeof split.nb);
+        memcpy(pp.cls_ns, split.ns, sizeof split.ns);
+        const hipFunction_t fn = d512 || split.split ? ctx->prefill[d512 ? 1 : 0] : ctx->prefill_whole;
+        if (int rc = launch(ctx, fn, dim3(split.blocks, a->Hkv, 1), dim3(512, 1, 1), pp, "prefill", true))
             return rc;
-        if (pp.nbig == 0) return G4A_OK;
-        // one 4-wave workgroup per (split block, dim half, kv head)
-        return launch(ctx, ctx->prefill_merge, dim3(2 * pp.nbig, a->Hkv, 1), dim3(256, 1, 1), pp, "prefill merge");
+        if (split.split == 0) return G4A_OK;
+        return launch(ctx, ctx->prefill_merge[d512 ? 1 : 0], dim3(split.split * (d512 ? 8 : 4), a->Hkv, 1),
+                      dim3(256, 1, 1), pp, "prefill merge");
     }
     // split-K flash-decode (+ combine)
     const uint32_t *qd = nullptr, *kd = nullptr;

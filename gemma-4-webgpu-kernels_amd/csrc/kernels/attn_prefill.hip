@@ -233,6 +233,36 @@ __device__ __forceinline__ void split_kv(const G4aSplitParams& p) {
     if (bad) *p.vflag = p.epoch;
 }
 
+// Workgroup `x` of a prefill launch: its query block, and which of the block's
+// ns shares of key tiles it takes (G4aPrefillParams::cls_nb).
+struct PfItem {
+    uint32_t blk, share, ns;
+};
+__device__ __forceinline__ PfItem pf_item(const G4aPrefillParams& p, uint32_t x) {
+    // unrolled, so that every argument it needs loads with the kernel's first: one
+    // more round trip to them is 1.5 us
+    uint32_t hi = (p.T + 7) / 8, base = 0, at = 0, my_hi = 0, ns = 1;
+#pragma unroll
+    for (uint32_t c = 0; c < G4A_PF_CLASSES; ++c) {  // classes past the last are empty
+        const uint32_t nb = p.cls_nb[c], n = nb * p.cls_ns[c];
+        if (x >= base && x < base + n) {
+            at = x - base;
+            my_hi = hi;
+            ns = p.cls_ns[c];
+        }
+        base += n;
+        hi -= nb;
+    }
+    return ns == 1 ? PfItem{my_hi - 1 - at, 0u, 1u} : PfItem{my_hi - 1 - at / ns, at % ns, ns};
+}
+
+// A wave's partial of a split block: O of its 16 rows x 256 columns in the
+// register layout (float4 (c * 4 + r) * 64 + lane holds row 4g + r's columns
+// 64c + 4rl .. +3), then l and m of the rows. 4 waves per slot at head_dim 256,
+// 8 (the lower half of the columns first) at 512.
+constexpr int PF_PART_O = 16 * 256;
+constexpr int PF_PART = PF_PART_O + 2 * 16;
+
 template <int DH>
 struct PairCfg {
     static constexpr int BK = 16;
@@ -255,7 +285,9 @@ struct PairCfg {
     static_assert(DH % 256 == 0, "rows are copied in 1 KiB pieces");
 };
 
-template <int DH>
+// SPLIT = false: no block is split (a full prompt's window: 0.7 us of 86 saved by
+// reading no class table).
+template <int DH, bool SPLIT>
 __device__ __forceinline__ void prefill_pair(const G4aPrefillParams& p) {
     using C = PairCfg<DH>;
     constexpr int BK = C::BK, KRS = C::KRS, RPW = C::RPW, NC = C::NC, QT = C::QT, CAP = C::CAP, SR = C::SR;
@@ -266,7 +298,8 @@ __device__ __forceinline__ void prefill_pair(const G4aPrefillParams& p) {
     const int rb = w & 3, par = w >> 2;
     const int g = lane >> 4, rl = lane & 15;
     const uint32_t kvh = blockIdx.y;
-    const uint32_t qb = blockIdx.x * 8;
+    const PfItem item = SPLIT ? pf_item(p, blockIdx.x) : PfItem{blockIdx.x, 0u, 1u};
+    const uint32_t qb = item.blk * 8;
     const uint32_t qw = qb + 2 * rb;
     const uint32_t h0 = kvh * 8;
     const size_t row_stride = (size_t)p.Hkv * DH;
@@ -292,8 +325,12 @@ __device__ __forceinline__ void prefill_pair(const G4aPrefillParams& p) {
     const int32_t wg_lo = key_lo(qb), wg_hi = key_hi(qlast);
     // tiles start on multiples of BK (the pre-split V quads are aligned to them);
     // keys of the first tile before wg_lo are masked like any invisible key
-    const int32_t wg_base = wg_lo & ~(BK - 1);
-    const uint32_t nt = wg_hi > wg_lo ? (uint32_t)((wg_hi - wg_base + BK - 1) / BK) : 0;
+    const int32_t blk_base = wg_lo & ~(BK - 1);
+    const uint32_t blk_nt = wg_hi > wg_lo ? (uint32_t)((wg_hi - blk_base + BK - 1) / BK) : 0;
+    // this workgroup's share of them: nt tiles from wg_base
+    const uint32_t t_begin = blk_nt * item.share / item.ns;
+    const int32_t wg_base = blk_base + (int32_t)(t_begin * BK);
+    const uint32_t nt = blk_nt * (item.share + 1) / item.ns - t_begin;
     const uint32_t nsteps = (nt + 1) / 2;
     // P.V from fp16 hi/lo splits of P and V unless some V value is outside their range
     const bool v16 = __builtin_amdgcn_readfirstlane(*p.vflag) != p.epoch;
@@ -731,6 +768,27 @@ __device__ __forceinline__ void prefill_pair(const G4aPrefillParams& p) {
         const float e0 = (m_ref == NEG_INF) ? 0.0f : expf(m_ref - M);
         const float e1 = (m1 == NEG_INF) ? 0.0f : expf(m1 - M);
         const float lt = l * e0 + l1 * e1;
+        if (SPLIT && item.ns > 1) {
+            // a share of a split block: its partial (O, l, m), in the register layout
+            float* const mine = p.part + (((size_t)kvh * p.part_slots + blockIdx.x) * 4 + rb) * PF_PART;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float f0 = __shfl(e0, 4 * g + r, 64), f1 = __shfl(e1, 4 * g + r, 64);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    float o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        o[e] = O[c][e][r] * f0 + mo_[((c * 4 + e) * 4 + r) * 64 + lane] * f1;
+                    reinterpret_cast<float4*>(mine)[(c * 4 + r) * 64 + lane] = make_float4(o[0], o[1], o[2], o[3]);
+                }
+            }
+            if (g == 0) {
+                mine[PF_PART_O + rl] = lt;
+                mine[PF_PART_O + 16 + rl] = M;
+            }
+            return;
+        }
         const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
         float a0[4], a1[4];
 #pragma unroll
@@ -769,9 +827,6 @@ __device__ __forceinline__ void prefill_pair(const G4aPrefillParams& p) {
 // candidate lists and l), and each wave runs P.V (fp16 hi/lo splits) and the
 // exact corrections for its own 256 output columns. Tiles stream into a 2-slot
 // LDS ring with global->LDS copies, one tile ahead.
-// Causal balance: a query block with more key tiles than the average runs as
-// two workgroups over the two halves of its tiles (p.nbig, see G4aPrefillParams);
-// each writes its partial (O, l, m) and prefill_merge combines them.
 template <int DH>
 struct DsplitCfg {
     static constexpr int BK = 16;
@@ -785,7 +840,6 @@ struct DsplitCfg {
     static constexpr int XS = 8 * 64 * 4;             // partial-score exchange [wave][lane][4]
     static constexpr int STAGE = (64 + 16) * 36;      // per-wave staging floats at the end (in the tile buffers)
     static constexpr int SMEM = 2 * TILE + XS + 8 * 2 * CAP + 8 * 16 + 8;  // ..., pair flags
-    static constexpr int PART_WAVE = NCH * 16 * 64 + 2 * 16;  // a wave's partial: O, then l and m of its rows
     static_assert(8 * STAGE <= 2 * TILE, "the end-of-kernel staging areas fit in the tile buffers");
     static_assert(BK * NPR == 8 * 4, "a tile is 64 pieces of 1 KiB: 8 per wave");
     static_assert(SMEM * 4 <= 160 * 1024, "LDS budget of a CU");
@@ -802,14 +856,8 @@ __device__ __forceinline__ void prefill_dsplit(const G4aPrefillParams& p) {
     const int rb = w & 3, dhf = w >> 2;
     const int g = lane >> 4, rl = lane & 15;
     const uint32_t kvh = blockIdx.y;
-    // work item: the two halves of each of the last nbig query blocks, then the
-    // other blocks, heaviest (latest queries) first
-    const uint32_t NB = (p.T + 7) / 8;
-    const uint32_t item = blockIdx.x;
-    const bool split = item < 2 * p.nbig;
-    const uint32_t half_id = split ? (item & 1u) : 0u;
-    const uint32_t blk = split ? NB - 1 - item / 2 : NB - 1 - p.nbig - (item - 2 * p.nbig);
-    const uint32_t qb = blk * 8;
+    const PfItem item = pf_item(p, blockIdx.x);
+    const uint32_t qb = item.blk * 8;
     const uint32_t qw = qb + 2 * rb;
     const uint32_t h0 = kvh * 8;
     const size_t row_stride = (size_t)p.Hkv * DH;
@@ -843,9 +891,9 @@ __device__ __forceinline__ void prefill_dsplit(const G4aPrefillParams& p) {
     // keys of the first tile before wg_lo are masked like any invisible key
     const int32_t wg_base = wg_lo & ~(BK - 1);
     const uint32_t nt = wg_hi > wg_lo ? (uint32_t)((wg_hi - wg_base + BK - 1) / BK) : 0;
-    // this workgroup's tiles [t_begin, t_end): all of them, or one half of a split block
-    const uint32_t t_begin = split && half_id ? nt / 2 : 0u;
-    const uint32_t t_end = split && !half_id ? nt / 2 : nt;
+    // this workgroup's share [t_begin, t_end) of them
+    const uint32_t t_begin = item.ns == 1 ? 0u : nt * item.share / item.ns;
+    const uint32_t t_end = item.ns == 1 ? nt : nt * (item.share + 1) / item.ns;
     const bool v16 = __builtin_amdgcn_readfirstlane(*p.vflag) != p.epoch;
     const float psc = v16 ? PF_PSCALE : 1.0f;  // scale of P, O and l (the f32 P.V path needs none)
     const bool wave_valid = qw < p.T;
@@ -1290,7 +1338,7 @@ __device__ __forceinline__ void prefill_dsplit(const G4aPrefillParams& p) {
     float l = l_part;
     l = g4a_col_sum4(l);
     // O row 4g + r' is query qw + row/8, head h0 + row%8; this wave's columns HD*dhf + 64c + 4rl + e
-    if (!split) {
+    if (item.ns == 1) {
         if (!wave_valid) return;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1307,88 +1355,120 @@ __device__ __forceinline__ void prefill_dsplit(const G4aPrefillParams& p) {
         }
         return;
     }
-    // ---- one half of a split block: its partial, in the wave's register layout ----
-    const uint32_t bi = kvh * p.nbig + (blk - (NB - p.nbig));  // split block of this kv head
-    float* const mine = p.part + ((size_t)(bi * 2 + half_id) * 8 + w) * C::PART_WAVE;
+    // ---- a share of a split block: its partial, in the wave's register layout ----
+    float* const mine = p.part + (((size_t)kvh * p.part_slots + blockIdx.x) * 8 + w) * PF_PART;
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mine[((c * 4 + e) * 4 + r) * 64 + lane] = O[c][e][r];
+        for (int c = 0; c < NCH; ++c)
+            reinterpret_cast<float4*>(mine)[(c * 4 + r) * 64 + lane] =
+                make_float4(O[c][0][r], O[c][1][r], O[c][2][r], O[c][3][r]);
     if (g == 0) {
-        mine[NCH * 16 * 64 + rl] = l;
-        mine[NCH * 16 * 64 + 16 + rl] = m_ref;
+        mine[PF_PART_O + rl] = l;
+        mine[PF_PART_O + 16 + rl] = m_ref;
     }
 }
 
-// Merge of the two halves of each split query block of prefill_dsplit:
-// workgroup = (split block, dim half, kv head), wave w = the producing waves'
-// (row block w, dim half); out = (O0 e^{m0-M} + O1 e^{m1-M}) / (l0 e^{m0-M} + l1 e^{m1-M}).
-// Every load of a thread is issued before the first use (the stores to `out`
-// would otherwise keep the compiler from moving later loads above them: one
-// memory round trip per 8 loads).
+// Merge of a split query block's shares: out = sum_s O_s e^{m_s - M} / sum_s l_s e^{m_s - M},
+// M = max_s m_s. Workgroup = (split block, one producing wave's 16 rows x 256 columns,
+// kv head). The rows' factors are worked out once per workgroup; then thread
+// (c, lane) sums its four rows' float4 over the shares, four shares' loads in
+// flight, the first four's from the start: bound by reading the partials once
+// (16 KiB per share and workgroup).
 template <int DH>
 __device__ __forceinline__ void prefill_merge(const G4aPrefillParams& p) {
-    using C = DsplitCfg<DH>;
-    constexpr int HD = C::HD, NCH = C::NCH;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int rb = tid >> 6, dhf = blockIdx.x & 1;
-    const int w = rb + 4 * dhf;  // the producing wave
+    constexpr int W = DH == 512 ? 8 : 4;  // waves per slot
+    __shared__ float fac[G4A_PF_MAX_SHARES][16];
+    const int tid = threadIdx.x, lane = tid & 63, c = tid >> 6;
     const int g = lane >> 4, rl = lane & 15;
-    const uint32_t kvh = blockIdx.y;
-    const uint32_t NB = (p.T + 7) / 8;
-    const uint32_t sb = blockIdx.x >> 1;
-    const uint32_t blk = NB - p.nbig + sb;
-    const uint32_t qw = blk * 8 + 2 * rb;
-    const uint32_t h0 = kvh * 8;
-    const uint32_t bi = kvh * p.nbig + sb;
-    const float* __restrict__ const p0 = p.part + ((size_t)(bi * 2 + 0) * 8 + w) * C::PART_WAVE;
-    const float* __restrict__ const p1 = p.part + ((size_t)(bi * 2 + 1) * 8 + w) * C::PART_WAVE;
-    float x0[4][NCH][4], x1[4][NCH][4], l0[4], m0[4], l1[4], m1[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = 4 * g + r;
-        l0[r] = p0[NCH * 16 * 64 + row];
-        m0[r] = p0[NCH * 16 * 64 + 16 + row];
-        l1[r] = p1[NCH * 16 * 64 + row];
-        m1[r] = p1[NCH * 16 * 64 + 16 + row];
-#pragma unroll
-        for (int c = 0; c < NCH; ++c)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int idx = ((c * 4 + e) * 4 + r) * 64 + lane;
-                x0[r][c][e] = p0[idx];
-                x1[r][c][e] = p1[idx];
-            }
+    const uint32_t kvh = blockIdx.y, w = blockIdx.x % W;
+    uint32_t y = blockIdx.x / W, hi = (p.T + 7) / 8, slot = 0, ns = 1;
+    for (uint32_t k = 0; k < p.ncls; ++k) {
+        const uint32_t nb = p.cls_nb[k];
+        ns = p.cls_ns[k];
+        if (y < nb) break;
+        y -= nb;
+        hi -= nb;
+        slot += nb * ns;
     }
+    slot += y * ns;
+    const uint32_t qw = (hi - 1 - y) * 8 + 2 * (w & 3);
+    if (qw >= p.T) return;
+    const size_t step = (size_t)W * PF_PART;  // floats between shares
+    const float* __restrict__ const src = p.part + (((size_t)kvh * p.part_slots + slot) * W + w) * PF_PART;
+    const float4* __restrict__ const o = reinterpret_cast<const float4*>(src) + c * 256 + lane;
+    float4 x[4][4];
+    auto load = [&](uint32_t s) {  // four shares (past the last: that one again)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[u][r] = o[min(s + u, ns - 1) * (step / 4) + r * 64];
+    };
+    load(0);
+    {
+        // row tid / 16's maxima and sums, 16 threads over its shares (all loads in flight)
+        constexpr int U = G4A_PF_MAX_SHARES / 16;
+        const int row = tid >> 4;
+        float m[U], l[U], M = NEG_INF, L = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t s = min((uint32_t)(tid & 15) + 16 * u, ns - 1);
+            m[u] = src[s * step + PF_PART_O + 16 + row];
+            l[u] = src[s * step + PF_PART_O + row];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) M = fmaxf(M, m[u]);
+        M = g4a_row_max16(M);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            m[u] = m[u] == NEG_INF ? 0.0f : expf(m[u] - M);
+            if ((uint32_t)(tid & 15) + 16 * u < ns) L += l[u] * m[u];
+        }
+        L = g4a_row_sum16(L);
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t s = (uint32_t)(tid & 15) + 16 * u;
+            if (s < ns) fac[s][row] = m[u] * inv;
+        }
+    }
+    __syncthreads();
+    float4 acc[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (uint32_t s = 0;;) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (s + u >= ns) break;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float f = fac[s + u][4 * g + r];
+                acc[r].x += x[u][r].x * f;
+                acc[r].y += x[u][r].y * f;
+                acc[r].z += x[u][r].z * f;
+                acc[r].w += x[u][r].w * f;
+            }
+        }
+        s += 4;
+        if (s >= ns) break;
+        load(s);
+    }
+    const uint32_t col = (DH == 512 ? 256 * (w >> 2) : 0) + 64 * c + 4 * rl;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int row = 4 * g + r;
         const uint32_t qi = qw + (row >> 3);
-        if (qi >= p.T) continue;
-        const float M = fmaxf(m0[r], m1[r]);
-        const float e0 = (m0[r] == NEG_INF) ? 0.0f : expf(m0[r] - M);
-        const float e1 = (m1[r] == NEG_INF) ? 0.0f : expf(m1[r] - M);
-        const float L = l0[r] * e0 + l1[r] * e1;
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        const float a0 = e0 * inv, a1 = e1 * inv;
-        float* orow = p.out + ((size_t)qi * p.Hq + h0 + (row & 7)) * DH + HD * dhf + 4 * rl;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = x0[r][c][e] * a0 + x1[r][c][e] * a1;
-            *reinterpret_cast<float4*>(orow + 64 * c) = make_float4(o[0], o[1], o[2], o[3]);
-        }
+        if (qi < p.T) *reinterpret_cast<float4*>(p.out + ((size_t)qi * p.Hq + kvh * 8 + (row & 7)) * DH + col) = acc[r];
     }
 }
 
 }  // namespace
 
 extern "C" {
-__global__ __launch_bounds__(512) void g4a_prefill2_d256(G4aPrefillParams p) { prefill_pair<256>(p); }
+__global__ __launch_bounds__(512) void g4a_prefill2_d256(G4aPrefillParams p) { prefill_pair<256, false>(p); }
+__global__ __launch_bounds__(512) void g4a_prefill2_split_d256(G4aPrefillParams p) { prefill_pair<256, true>(p); }
 __global__ __launch_bounds__(512) void g4a_prefill2_d512(G4aPrefillParams p) { prefill_dsplit<512>(p); }
+__global__ __launch_bounds__(256) void g4a_prefill_merge_d256(G4aPrefillParams p) { prefill_merge<256>(p); }
 __global__ __launch_bounds__(256) void g4a_prefill_merge_d512(G4aPrefillParams p) { prefill_merge<512>(p); }
 __global__ __launch_bounds__(256) void g4a_split_kv(G4aSplitParams p) { split_kv(p); }
 }

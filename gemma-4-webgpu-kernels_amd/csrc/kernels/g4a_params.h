@@ -101,6 +101,11 @@ struct G4aGenericParams {
     float scale, softcap;
 };
 
+// Most classes of split query blocks of a prefill launch.
+constexpr uint32_t G4A_PF_CLASSES = 14;
+// Most workgroups of one query block.
+constexpr uint32_t G4A_PF_MAX_SHARES = 128;
+
 // Query-tiled causal / sliding-window prefill over contiguous positions:
 // query i has position q_pos0 + i, key j has position k_pos0 + j; group of 8
 // query heads per kv head; Dh == Dv in {256, 512}; no soft-cap.
@@ -120,13 +125,17 @@ struct G4aPrefillParams {
     uint32_t split0, split_n, epoch;
     float scale;
     float tau;             // rescoring band: keys whose estimated score is within tau of the row maximum are rescored exactly
-    // head_dim 512 causal balance: the last `nbig` query blocks (8 queries each)
-    // run as two workgroups over the two halves of their key tiles; each half
-    // writes its partial (O, l, m) to `part` and g4a_prefill_merge_d512 merges
-    // them. Workgroup i runs the split halves first, then the other blocks,
-    // heaviest first (so heavy work starts first).
+    // Split query blocks. Blocks of 8 queries fall into ncls classes, the latest
+    // (under a causal mask the heaviest) blocks first: class c holds cls_nb[c]
+    // blocks of cls_ns[c] workgroups each, over equal shares of the block's
+    // 16-key tiles. cls_ns does not increase with c, so the workgroups of split
+    // blocks are the launch's first, and workgroup i of them writes its partial
+    // (O, l, m) to slot i of `part`; g4a_prefill_merge_d* merges a block's slots.
     float* part;
-    uint32_t nbig;
+    uint32_t part_slots;  // slots per kv head
+    uint32_t ncls;
+    uint32_t cls_nb[G4A_PF_CLASSES];
+    uint32_t cls_ns[G4A_PF_CLASSES];
 };
 
 // Pre-split keys for the head_dim 256 prefill: keys [k0, k0 + nkeys) (logical,
