@@ -130,6 +130,8 @@ struct g4a_ctx {
     hipFunction_t linear_words[3][3][3] = {};  // [bits 2/4/8][(MT, RU) = (1, 2), (1, 8), (4, 4)][mode]
     hipFunction_t linear_elem[3] = {};         // [mode]
     hipFunction_t linear_mfma[3][2][3] = {};   // [bits 2/4/8][64 / 128 weight rows per tile][mode]: M >= 16
+    hipFunction_t linear_mm[4][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
+    hipFunction_t split_x[3] = {};             // [bits 2/4/8]: the split
     hipFunction_t linear_i8[3][2] = {};        // [bits 2/4/8][M = 1, 2]: int8 matrix cores, mode 0
     // G4A_LINEAR_I8=0 keeps M <= 2 projections off the int8 matrix-core kernel,
     // =1 sends every eligible one there (for comparisons); unset: by weight size
@@ -751,6 +753,17 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
                     snprintf(name, sizeof name, "g4a_linear_q_mfma_b%d_n%d_mode%d", bits[b], t ? 128 : 64, m);
                     if (int rc = get_fn(ctx, &ctx->linear_mfma[b][t][m], name)) return bail(rc);
                 }
+        }
+        for (int b = 0; b < 3; ++b) {
+            char name[64];
+            for (int m = 0; m < 3; ++m) {
+                for (int f = 0; f < 4; ++f) {
+                    snprintf(name, sizeof name, "g4a_linear_mm_%d_b%d_mode%d", f, bits[b], m);
+                    if (int rc = get_fn(ctx, &ctx->linear_mm[f][b][m], name)) return bail(rc);
+                }
+            }
+            snprintf(name, sizeof name, "g4a_split_x_b%d", bits[b]);
+            if (int rc = get_fn(ctx, &ctx->split_x[b], name)) return bail(rc);
         }
         for (int b = 0; b < 3; ++b)
             for (int m = 0; m < 2; ++m) {
@@ -1496,6 +1509,9 @@ int norm_rope_launch(g4a_ctx* ctx, G4aNormRopeSeg* segs, uint32_t nseg, uint32_t
 constexpr size_t LINEAR_LDS_BYTES = 64 << 10;
 // Activation rows from which a projection runs on the matrix cores.
 constexpr uint32_t LINEAR_MFMA_MIN_M = 16;
+// Row length above which those calls split x ahead (linear_mm_*): at K = 256 the
+// split's launch costs more than it saves (M = 64, N = 1536: 7.8 us without, 10 with).
+constexpr uint32_t LINEAR_MM_MIN_K = 256;
 // Packed weight bytes from which an M <= 2 projection runs on the int8 matrix
 // cores (below it the word kernel's shorter start wins; both are at the
 // dispatch floor there).
@@ -1599,6 +1615,85 @@ LinearChoice choose_linear(const g4a_ctx* ctx, int mode, const g4a_qweight* w, c
     return c;
 }
 
+// The linear_mm form of a call: the one whose workgroups take the least time,
+// ceil(workgroups / CUs) of them after one another on a CU, at `step` us per 64 k
+// and `fixed` us per workgroup (measured with every CU busy, 4-bit; 8-bit weights'
+// loads take the k-split forms and the one-wave-a-SIMD tile longer). The choice is
+// within 10 % of the best form over M = 16 .. 2048 of [2048, 1536], [1536, 6144],
+// [1536, 12288] and gate + up [6144, 1536], [12288, 1536] weights at 2, 4 and 8 bits.
+struct MmForm {
+    int form;
+    uint32_t rows, toks, threads;  // weight rows (of each weight) and tokens of a workgroup
+    float step[2], fixed, wide;    // mode 0 and 2, mode 1; factor at 8 bits
+};
+constexpr MmForm MM_FORMS[4] = {
+    {0, 256, 128, 512, {1.85f, 1.85f}, 4.0f, 1.0f},
+    {1, 128, 128, 256, {1.05f, 1.05f}, 4.0f, 1.45f},
+    {2, 64, 32, 512, {0.19f, 0.33f}, 2.0f, 1.7f},
+    {3, 32, 32, 512, {0.131f, 0.18f}, 1.1f, 1.4f},
+};
+
+MmForm linear_mm_choose(const g4a_ctx* ctx, int mode, int bi, uint32_t M, uint32_t N, uint32_t K, bool tiles) {
+    const uint64_t cus = uint64_t(std::max(ctx->cu_count, 1));
+    MmForm best = MM_FORMS[3];
+    float least = 3.0e38f;
+    for (MmForm f : MM_FORMS) {
+        if (f.form <= 1 && !tiles) continue;
+        if (mode == 1 && f.form <= 1) f.rows /= 2;  // the tiles hold rows of both weights
+        const uint64_t wgs = uint64_t((N + f.rows - 1) / f.rows) * ((M + f.toks - 1) / f.toks);
+        const float t = float((wgs + cus - 1) / cus) *
+                        (f.step[mode == 1] * (bi == 2 ? f.wide : 1.0f) * float(K / 64) + f.fixed);
+        if (t < least) least = t, best = f;
+    }
+    return best;
+}
+
+// Rows of x that linear_mm_launch splits at a time (a multiple of its 128-row
+// tiles; the split copy is as large as x: 256 MiB at most), and the bytes of a
+// split of `rows` rows: the parts, then the scales.
+uint32_t linear_mm_rows(uint32_t M, uint32_t K) {
+    const uint64_t most = std::max<uint64_t>(128, (uint64_t(256) << 20) / (uint64_t(K) * 4) / 128 * 128);
+    return uint32_t(std::min<uint64_t>(most, M));
+}
+size_t split_x_bytes(uint32_t rows, uint32_t K) {
+    return size_t(rows + 31) / 32 * 32 * (size_t(K) + (K + 255) / 256) * sizeof(float);
+}
+
+// Whether the context has, or can get, the memory of a split x: not in a graph
+// capture whose workspace would grow, nor when the device is out of memory (the
+// call then takes linear_q_mfma, which needs none).
+bool linear_mm_fits(g4a_ctx* ctx, const G4aLinearParams& p) {
+    const size_t need = split_x_bytes(linear_mm_rows(p.M, p.K), p.K);
+    if (need <= ctx->workspace_bytes) return true;
+    if (ctx->capturing) return false;
+    const std::string err = ctx->err;
+    if (ensure_workspace(ctx, need) == G4A_OK) return true;
+    ctx->err = err;
+    return false;
+}
+
+int linear_mm_launch(g4a_ctx* ctx, int mode, int bi, const G4aLinearParams& p) {
+    const uint32_t most = linear_mm_rows(p.M, p.K), nseg = (p.K + 255) / 256;
+    for (uint32_t m0 = 0; m0 < p.M; m0 += most) {
+        const uint32_t M = std::min(most, p.M - m0), nblk = (M + 31) / 32;
+        float* const xs = static_cast<float*>(ctx->workspace);
+        float* const xscale = xs + size_t(nblk) * 32 * p.K;
+        G4aSplitXParams sp{p.x + size_t(m0) * p.K, xs, xscale, M, p.K};
+        if (int rc = launch(ctx, ctx->split_x[bi], dim3(nseg, nblk, 1), dim3(256, 1, 1), sp, "split x")) return rc;
+        G4aLinearMmParams q{p.wb, p.wb2, xs, xscale, p.s, p.s2, p.b ? p.b + size_t(m0) * p.b_stride : nullptr,
+                            p.y + size_t(m0) * p.N, M, p.N, p.K, p.row_bytes, p.b_stride, p.b_off,
+                            p.signed_i8 ? 0x80808080u : 0u};
+        // (the tiles copy weights to LDS 16 bytes at a time)
+        const bool tiles = ((reinterpret_cast<uintptr_t>(p.wb) | reinterpret_cast<uintptr_t>(p.wb2)) & 15) == 0;
+        const MmForm f = linear_mm_choose(ctx, mode, bi, M, p.N, p.K, tiles);
+        const int rc = launch(ctx, ctx->linear_mm[f.form][bi][mode], dim3((p.N + f.rows - 1) / f.rows,
+                              (M + f.toks - 1) / f.toks, 1), dim3(f.threads, 1, 1), q,
+                              "quantised linear (matrix cores)", true);
+        if (rc) return rc;
+    }
+    return G4A_OK;
+}
+
 int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qweight* w2, const float* x,
                     const float* b, uint32_t b_stride, uint32_t b_off, float* y, uint32_t M) {
     if (!ctx) return fail(ctx, G4A_E_ARG, "null ctx");
@@ -1641,6 +1736,7 @@ int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qwei
         // or x 64 rows when the larger tile would leave fewer than 2 workgroups per CU
         p.wb = static_cast<const uint8_t*>(w->qbytes);
         p.wb2 = mode == 1 ? static_cast<const uint8_t*>(w2->qbytes) : nullptr;
+        if (w->K > LINEAR_MM_MIN_K && linear_mm_fits(ctx, p)) return linear_mm_launch(ctx, mode, bi, p);
         const int wide = ch.wide;
         const uint32_t gx = wide ? (w->N + 127) / 128 : (w->N + 63) / 64;
         for (uint32_t m0 = 0; m0 < M; m0 += 65535u * 64) {

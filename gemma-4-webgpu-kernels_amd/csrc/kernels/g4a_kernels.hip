@@ -5,4 +5,5 @@
 #include "attn_prefill.hip"
 #include "norm_rope.hip"
 #include "linear_q.hip"
+#include "linear_mm.hip"
 #include "elementwise.hip"

@@ -239,6 +239,31 @@ struct G4aLinearParams {
     uint32_t nsplit, dh, hq;
 };
 
+// Activations split into scaled fp16 hi/lo parts ahead of linear_mm_* (layout: split_x).
+struct G4aSplitXParams {
+    const float* x;   // [M, K], K a multiple of 64
+    void* xs;         // ceil(M / 32) * 32 * K * 4 bytes
+    float* xscale;    // [ceil(M / 32)][ceil(K / 256)][32]
+    uint32_t M, K;
+};
+
+// Quantised projection over split activations (g4a_linear_mm_*): modes, weights
+// and epilogues as G4aLinearParams.
+struct G4aLinearMmParams {
+    const uint8_t* wb;
+    const uint8_t* wb2;
+    const void* xs;
+    const float* xscale;
+    const float* s;
+    const float* s2;
+    const float* b;
+    float* y;
+    uint32_t M, N, K;
+    uint32_t row_bytes;
+    uint32_t b_stride, b_off;
+    uint32_t xm;  // 8-bit fields: the mask turning them into offset binary
+};
+
 // Split counts up to which a decode step's output projection merges the split
 // partials itself (mode 3), and the query heads it takes.
 constexpr uint32_t G4A_FUSE_MAX_SPLITS = 16;

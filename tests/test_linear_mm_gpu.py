@@ -1,0 +1,107 @@
+"""Projections of 16 and more rows on split activations (linear_mm_*): every form
+(128-token tiles of 256 and 128 rows, 32-token k-split blocks of 64 and 32 rows)
+at ragged edges of its tiles and steps, every weight format and epilogue, against
+the CPU oracle within the bound of another f32 summation order
+(2e-6 * sum |x w| + 1e-7 per output, as tests/test_linear_gpu.py derives it);
+activations far apart in scale within a row, whose segments scale apart; rows
+holding an inf or NaN; and a capture on a context whose workspace is too small
+for the split, which runs the kernel that needs none."""
+import numpy as np
+import pytest
+
+import g4a
+import g4a.synth as synth
+import oracle
+from test_linear_gpu import Dev, _bound, _check_fused, _check_sum, _qw
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("op,N,K,M,bits,signed", [
+    ("linear", 33, 320, 16, 4, False),       # k-split, fewer steps than waves, a ragged 32-row block
+    ("linear", 2050, 576, 33, 2, False),     # a segment of one step, N not a multiple of 4
+    ("linear", 700, 1536, 97, 8, True),
+    ("linear", 700, 1536, 97, 8, False),
+    ("gelu_cols", 95, 1600, 40, 4, False),
+    ("geglu", 100, 448, 65, 4, False),
+    ("geglu", 130, 1536, 31, 2, False),
+    ("linear", 4100, 320, 1030, 4, False),   # tiles, the last of each ragged
+    ("geglu", 3100, 320, 700, 2, False),
+    ("geglu", 1050, 320, 900, 8, True),
+    ("gelu_cols", 4099, 320, 600, 4, False),
+])
+def test_forms_match_the_oracle(ctx, op, N, K, M, bits, signed):
+    name = f"{op} N={N} K={K} M={M} b{bits}{'s' if signed else ''}"
+    print(f"[gpu] {name}", flush=True)
+    w, x = _qw(1, N, K, bits, signed, None), synth.normal_f32(2, 1, M * K).reshape(M, K)
+    with Dev(ctx) as d:
+        dw, dx, y = d.w(w), d.arr(x), d.empty((M, N))
+        if op == "linear":
+            ctx.linear_q(dw, dx.ptr, y.ptr, M)
+            _check_sum(y.to_host(), oracle.linear_q(x, w), _bound(x, w), name)
+        elif op == "geglu":
+            w2 = _qw(3, N, K, bits, signed, None)
+            ctx.linear_q_geglu(dw, d.w(w2), dx.ptr, y.ptr, M)
+            _check_fused(y.to_host(), x, w, w2, None, 0, name)
+        else:
+            b = synth.normal_f32(4, 2, M * (N + 5)).reshape(M, N + 5)
+            ctx.linear_q_gelu_mul_cols(dw, dx.ptr, d.arr(b).ptr, N + 5, 3, y.ptr, M)
+            _check_fused(y.to_host(), x, w, None, b, 3, name)
+
+
+@pytest.mark.parametrize("bits,signed", [(4, False), (8, True), (2, False)])
+def test_weights_at_eight_byte_alignment(ctx, bits, signed):
+    # 8 bytes past a 16-byte boundary: the tiles' 16-byte weight copies do not run
+    N, K, M = 4096, 320, 700
+    w, x = _qw(9, N, K, bits, signed, None), synth.normal_f32(10, 1, M * K).reshape(M, K)
+    print(f"[gpu] b{bits}", flush=True)
+    raw = ctx.upload(np.concatenate([np.zeros(8, np.uint8), np.ascontiguousarray(w.qbytes, np.uint8).ravel()]))
+    with Dev(ctx) as d:
+        dw, y = d.w(w), d.empty((M, N))
+        args = g4a.QWeightArgs(raw.ptr + 8, dw.args.scales, N, K, bits, int(signed), K)
+        ctx.linear_q(g4a.DeviceQWeight(args, None, None), d.arr(x).ptr, y.ptr, M)
+        _check_sum(y.to_host(), oracle.linear_q(x, w), _bound(x, w), f"b{bits}")
+    raw.free()
+
+
+@pytest.mark.parametrize("M", [20, 400])
+def test_scales_apart_and_non_finite_rows(ctx, M):
+    N, K = 2048, 1024
+    w, x = _qw(5, N, K, 4, False, None), synth.normal_f32(6, 1, M * K).reshape(M, K).copy()
+    x[0, :256] *= np.float32(1e30)
+    x[1, 256:512] *= np.float32(1e-30)
+    x[2] *= np.float32(1e-38)
+    x[3, ::2] *= np.float32(2.0 ** -20)
+    x[4] = 0.0
+    x[5, 700] = np.inf
+    x[6, 3] = np.nan
+    print(f"[gpu] M={M}", flush=True)
+    fine = [m for m in range(M) if m not in (5, 6)]
+    with Dev(ctx) as d:
+        y = d.empty((M, N))
+        ctx.linear_q(d.w(w), d.arr(x).ptr, y.ptr, M)
+        got = y.to_host()
+    # the bound's absolute part is for rows of about unit values: compare per row in units of its largest
+    unit = np.maximum(np.abs(x[fine]).max(1, keepdims=True), np.float32(1e-45)).astype(np.float64)
+    want = oracle.linear_q(x[fine], w)
+    assert np.all(np.abs(got[fine].astype(np.float64) - want) <= 2e-6 * _bound(x[fine], w) + 1e-7 * unit)
+    assert not got[4].any()
+    assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
+
+
+def test_capture_without_room_for_the_split(ctx):
+    N, K, M = 256, 1536, 3000  # the split takes 19 MB; a context starts with no workspace
+    w, x = _qw(7, N, K, 4, False, None), synth.normal_f32(8, 1, M * K).reshape(M, K)
+    with g4a.Context(0) as own, Dev(own) as d:
+        dw, dx, y = d.w(w), d.arr(x), d.empty((M, N))
+        print("[gpu] capture", flush=True)
+        own.capture_begin()
+        own.linear_q(dw, dx.ptr, y.ptr, M)
+        graph = own.capture_end()
+        want, bound = oracle.linear_q(x[:100], w), _bound(x[:100], w)
+        for _ in range(2):
+            graph.launch()
+            _check_sum(y.to_host()[:100], want, bound, "replay")
+            own.linear_q(dw, dx.ptr, y.ptr, M)  # the workspace grows between the replays
+            _check_sum(y.to_host()[:100], want, bound, "eager")
+        graph.free()
