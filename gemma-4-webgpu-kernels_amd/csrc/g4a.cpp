@@ -131,6 +131,7 @@ struct g4a_ctx {
     hipFunction_t linear_elem[3] = {};         // [mode]
     hipFunction_t linear_mfma[3][2][3] = {};   // [bits 2/4/8][64 / 128 weight rows per tile][mode]: M >= 16
     hipFunction_t linear_mm[4][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
+    hipFunction_t linear_few[2][3][3] = {};    // [16 / 64 rows a workgroup][bits][mode]: at most 16 activation rows
     hipFunction_t split_x[3] = {};             // [bits 2/4/8]: the split
     hipFunction_t linear_i8[3][2] = {};        // [bits 2/4/8][M = 1, 2]: int8 matrix cores, mode 0
     // G4A_LINEAR_I8=0 keeps M <= 2 projections off the int8 matrix-core kernel,
@@ -757,6 +758,10 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
         for (int b = 0; b < 3; ++b) {
             char name[64];
             for (int m = 0; m < 3; ++m) {
+                for (int r = 0; r < 2; ++r) {
+                    snprintf(name, sizeof name, "g4a_linear_mm_few_r%d_b%d_mode%d", r ? 2 : 1, bits[b], m);
+                    if (int rc = get_fn(ctx, &ctx->linear_few[r][b][m], name)) return bail(rc);
+                }
                 for (int f = 0; f < 4; ++f) {
                     snprintf(name, sizeof name, "g4a_linear_mm_%d_b%d_mode%d", f, bits[b], m);
                     if (int rc = get_fn(ctx, &ctx->linear_mm[f][b][m], name)) return bail(rc);
@@ -1516,6 +1521,12 @@ constexpr uint32_t LINEAR_MM_MIN_K = 256;
 // cores (below it the word kernel's shorter start wins; both are at the
 // dispatch floor there).
 constexpr uint64_t LINEAR_I8_MIN_BYTES = 16ull << 20;
+// Packed weight bytes from which 3 .. 8 rows run there too, two at a time, and the
+// most rows that do.
+constexpr uint64_t LINEAR_I8_PAIRS_MIN_BYTES = 64ull << 20;
+constexpr uint32_t LINEAR_I8_PAIRS_MAX_M = 8;
+// Most activation rows of the kernel that splits them in registers (linear_mm_few).
+constexpr uint32_t LINEAR_FEW_MAX_M = 16;
 
 // Grid of a grid-stride elementwise launch over n items.
 dim3 ew_grid(g4a_ctx* ctx, size_t n) {
@@ -1560,8 +1571,8 @@ int check_qweight(g4a_ctx* ctx, const g4a_qweight* w, const char* what) {
 // decides it (g4a_attention_linear_q asks it too, so the projection it merges a
 // decode step's partials into is the one the plain call would run).
 struct LinearChoice {
-    enum Kind { MFMA, I8, ELEM, WORDS } kind = ELEM;
-    int wide = 0;       // MFMA: 128-row tiles
+    enum Kind { MFMA, FEW, I8, ELEM, WORDS } kind = ELEM;
+    int wide = 0;       // MFMA without a split x: 128-row tiles; FEW: 32 weight rows a workgroup, else 16
     int variant = 0;    // WORDS: (MT, RU) = (1, 2), (1, 8), (4, 4)
     int MT = 1, RU = 2;
     bool half = false;  // WORDS: 2-bit rows of an odd multiple of 32 words, two rows per wave
@@ -1578,17 +1589,38 @@ LinearChoice choose_linear(const g4a_ctx* ctx, int mode, const g4a_qweight* w, c
     const bool aligned = (qa & 3) == 0 && (qa2 & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     const bool aligned8 = aligned && (qa & 7) == 0 && (qa2 & 7) == 0;
     const uint64_t cus = uint64_t(std::max(ctx->cu_count, 1));
-    if (M >= LINEAR_MFMA_MIN_M && w->K % 64 == 0 && scale_stride == 1 && aligned8) {
+    const bool mm_ok = w->K % 64 == 0 && scale_stride == 1 && aligned8;
+    const uint64_t weight_bytes = uint64_t(w->N) * row_bytes;
+    const bool i8_ok = mode == 0 && scale_stride == 1 && row_bytes % G4A_LI8_UNIT_BYTES == 0 && w->K % 64 == 0 &&
+                       uint64_t(w->K / 64) * 1024 <= LINEAR_LDS_BYTES && (qa & 15) == 0;
+    // a weight whose read alone is most of a pass (an output head): two rows a pass
+    // up to 8 rows (23 us each at 100 MB; 93 us as words for 4 rows, 107 as matrix-core
+    // blocks for 16), the blocks past them
+    const bool huge = i8_ok && mm_ok && ctx->linear_i8_use != 0 && weight_bytes >= LINEAR_I8_PAIRS_MIN_BYTES;
+    if (i8_ok && (M <= 2 ? ctx->linear_i8_use == 1 || (ctx->linear_i8_use < 0 && weight_bytes >= LINEAR_I8_MIN_BYTES)
+                         : huge && M <= LINEAR_I8_PAIRS_MAX_M)) {
+        c.kind = LinearChoice::I8;
+        return c;
+    }
+    // 2 .. 16 rows with x split in registers. Against the word kernel's passes of 4
+    // rows, us: [2048, 1536] M = 2 5.7 -> 4.7, M = 12 7.2 -> 5.8; gate + up
+    // [6144, 1536] M = 12 19.0 -> 9.8; [1536, 6144] M = 12 19.3 -> 14.7 but M = 4
+    // 9.2 -> 10.8, [32768, 1536] M = 8 22.7 -> 17.0 but M = 4 14.0 -> 15.1: long rows
+    // (few workgroups) and tall weights take it past one such pass. At 16 rows the
+    // blocks over a split x are level on long rows and tall weights.
+    if (mm_ok && M >= 2 && M <= LINEAR_FEW_MAX_M && !huge) {
+        const bool tall = w->N >= 16384, wide = w->K >= 6144;
+        if (M == LINEAR_FEW_MAX_M ? w->K <= 4096 && w->N <= 8192 : M > 4 || (!tall && !wide)) {
+            c.kind = LinearChoice::FEW;
+            // 32 rows a workgroup for tall weights, and where both of mode 1's weights fill the CUs once
+            c.wide = mode == 1 ? (w->N + 31) / 32 <= cus : tall;
+            return c;
+        }
+    }
+    if (mm_ok && (M >= LINEAR_MFMA_MIN_M || (huge && M > LINEAR_I8_PAIRS_MAX_M))) {
         c.kind = LinearChoice::MFMA;
         const uint64_t tiles128 = uint64_t((w->N + 127) / 128) * ((M + 63) / 64);
         c.wide = tiles128 >= 2 * cus ? 1 : 0;
-        return c;
-    }
-    const uint64_t weight_bytes = uint64_t(w->N) * row_bytes;
-    const bool i8_ok = mode == 0 && M <= 2 && scale_stride == 1 && row_bytes % G4A_LI8_UNIT_BYTES == 0 &&
-                       w->K % 64 == 0 && uint64_t(w->K / 64) * 1024 <= LINEAR_LDS_BYTES && (qa & 15) == 0;
-    if (i8_ok && (ctx->linear_i8_use == 1 || (ctx->linear_i8_use < 0 && weight_bytes >= LINEAR_I8_MIN_BYTES))) {
-        c.kind = LinearChoice::I8;
         return c;
     }
     const uint64_t vpw = 32 / w->bits, words_per_row = uint64_t(w->K) * w->bits / 32;
@@ -1680,7 +1712,7 @@ int linear_mm_launch(g4a_ctx* ctx, int mode, int bi, const G4aLinearParams& p) {
         float* const xscale = xs + size_t(nblk) * 32 * p.K;
         G4aSplitXParams sp{p.x + size_t(m0) * p.K, xs, xscale, M, p.K};
         if (int rc = launch(ctx, ctx->split_x[bi], dim3(nseg, nblk, 1), dim3(256, 1, 1), sp, "split x")) return rc;
-        G4aLinearMmParams q{p.wb, p.wb2, xs, xscale, p.s, p.s2, p.b ? p.b + size_t(m0) * p.b_stride : nullptr,
+        G4aLinearMmParams q{p.wb, p.wb2, xs, xscale, nullptr, p.s, p.s2, p.b ? p.b + size_t(m0) * p.b_stride : nullptr,
                             p.y + size_t(m0) * p.N, M, p.N, p.K, p.row_bytes, p.b_stride, p.b_off,
                             p.signed_i8 ? 0x80808080u : 0u};
         // (the tiles copy weights to LDS 16 bytes at a time)
@@ -1731,6 +1763,15 @@ int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qwei
     // sub-byte fields are offset binary: flipping each field's top bit makes it two's complement
     p.xm = w->signed_i8 ? 0u : w->bits == 4 ? 0x88888888u : w->bits == 2 ? 0xAAAAAAAAu : 0x80808080u;
     const int bi = w->bits == 2 ? 0 : w->bits == 4 ? 1 : 2;
+    if (ch.kind == LinearChoice::FEW) {
+        const G4aLinearMmParams q{static_cast<const uint8_t*>(w->qbytes),
+                                  mode == 1 ? static_cast<const uint8_t*>(w2->qbytes) : nullptr, nullptr, nullptr, x, p.s,
+                                  p.s2, p.b, p.y, M, p.N, p.K, p.row_bytes, p.b_stride, p.b_off,
+                                  p.signed_i8 ? 0x80808080u : 0u};
+        const uint32_t rows = ch.wide ? 32 : 16;
+        return launch(ctx, ctx->linear_few[ch.wide][bi][mode], dim3((w->N + rows - 1) / rows, 1, 1), dim3(512, 1, 1), q,
+                      "quantised linear (few rows)", true);
+    }
     if (ch.kind == LinearChoice::MFMA) {
         // 64 activation rows x 128 weight rows per workgroup on the matrix cores,
         // or x 64 rows when the larger tile would leave fewer than 2 workgroups per CU
@@ -1759,8 +1800,16 @@ int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qwei
         const uint64_t waves = G4A_LI8_THREADS / 64, chunks = (uint64_t(w->N) + 31) / 32;
         const uint64_t cap = uint64_t(std::max(ctx->cu_count, 1)) * (16 / waves);
         const uint32_t gx = uint32_t(std::max<uint64_t>(1, std::min(cap, (chunks + waves - 1) / waves)));
-        return launch(ctx, ctx->linear_i8[bi][M - 1], dim3(gx, 1, 1), dim3(G4A_LI8_THREADS, 1, 1), p,
-                      "quantised linear (int8 matrix cores)", true, unsigned(w->K / 64 * 1024));
+        for (uint32_t m0 = 0; m0 < M; m0 += 2) {
+            G4aLinearParams q = p;
+            q.x = x + size_t(m0) * w->K;
+            q.y = y + size_t(m0) * w->N;
+            q.M = std::min<uint32_t>(2, M - m0);
+            if (int rc = launch(ctx, ctx->linear_i8[bi][q.M - 1], dim3(gx, 1, 1), dim3(G4A_LI8_THREADS, 1, 1), q,
+                                "quantised linear (int8 matrix cores)", true, unsigned(w->K / 64 * 1024)))
+                return rc;
+        }
+        return G4A_OK;
     }
     // the word kernel's activation rows, zero-padded to whole wave strides of words
     const uint64_t vpw = 32 / w->bits, words_per_row = uint64_t(w->K) * w->bits / 32;

@@ -254,6 +254,7 @@ struct G4aLinearMmParams {
     const uint8_t* wb2;
     const void* xs;
     const float* xscale;
+    const float* x;  // linear_mm_few: [M, K] itself
     const float* s;
     const float* s2;
     const float* b;

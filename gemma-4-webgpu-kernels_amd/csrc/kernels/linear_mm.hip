@@ -410,7 +410,7 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
         float sc[TB];
     };
     auto load = [&](Step& s, uint32_t st) {
-        st = min(st, nsteps - 1);
+        if (st >= nsteps) return;  // (the step index is the wave's: no divergence)
 #pragma unroll
         for (int q = 0; q < NR; ++q) mm_load_w<BITS>(wp[q] + (size_t)st * 8 * BITS, s.w[q]);
 #pragma unroll
@@ -502,6 +502,184 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
     }
 }
 
+// A lane's words of a 64-k step for v_mfma_f32_16x16x32_f16 (16 k of a row), and
+// the 8 fields of its MFMA step i (0, 1) in the order of mm_k.
+template <int BITS>
+__device__ __forceinline__ void mm_load_w16(const uint8_t* src, uint32_t (&w)[BITS / 2]) {
+    if constexpr (BITS == 2) {
+        w[0] = *reinterpret_cast<const uint32_t*>(src);
+    } else if constexpr (BITS == 4) {
+        const uint2 v = *reinterpret_cast<const uint2*>(src);
+        w[0] = v.x;
+        w[1] = v.y;
+    } else {
+        typedef uint32_t u4a8 __attribute__((ext_vector_type(4), aligned(8)));
+        const u4a8 v = *reinterpret_cast<const u4a8*>(src);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = v[e];
+    }
+}
+// Four lanes of a row (g = lane / 16) hold 16 adjacent k each, while x is read with
+// four adjacent k per lane (whole 64-byte pieces per load): trade words across the
+// lanes so that lane g holds k = 16 j + 4 g .. + 3 for j = 0 .. 3. Fields of the
+// result: 8-bit word j; else word i holds j = i in its lower and i + 2 in its upper half.
+__device__ __forceinline__ void mm_swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void mm_swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+template <int BITS>
+__device__ __forceinline__ void mm_spread(const uint32_t (&w)[BITS / 2], uint32_t (&o)[BITS == 8 ? 4 : 2]) {
+    if constexpr (BITS == 8) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = w[e];
+        mm_swap32(o[0], o[2]);
+        mm_swap32(o[1], o[3]);
+        mm_swap16(o[0], o[1]);
+        mm_swap16(o[2], o[3]);
+    } else if constexpr (BITS == 4) {
+        uint32_t a = w[0], b = w[1];
+        mm_swap32(a, b);
+        o[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);  // lower halves
+        o[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);  // upper halves
+        mm_swap16(o[0], o[1]);
+    } else {
+        uint32_t a = w[0], b = w[0] >> 16;
+        mm_swap32(a, b);
+        o[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        o[1] = o[0] >> 8;
+        mm_swap16(o[0], o[1]);
+    }
+}
+// The 8 fields of MFMA step i (0, 1) of a 64-k step: position pos holds j, e as mm_few_x.
+template <int BITS>
+__device__ __forceinline__ mm_h8 mm_few_frag(const uint32_t (&o)[BITS == 8 ? 4 : 2], int i, uint32_t xm) {
+    uint32_t t[BITS];
+#pragma unroll
+    for (int e = 0; e < BITS; ++e) t[e] = o[e % (BITS == 8 ? 4 : 2)];
+    return mm_frag<BITS>(t, BITS == 2 ? 2 * i : i, xm);
+}
+// Index 4 j + e of that position's x.
+template <int BITS>
+__device__ __forceinline__ constexpr int mm_few_x(int i, int pos) {
+    return BITS == 8 ? 8 * i + pos : 4 * (i + 2 * (pos & 1)) + pos / 2;
+}
+
+// 16 rows of x or fewer (a serving batch's step): workgroup = 16 RB weight rows (of
+// each weight), 8 waves taking every eighth 64-k step, x split in registers by the
+// wave that uses it (a launch ahead for it would cost 3 us), one scale per token and
+// step; the waves' sums added through LDS in order. Bound by latency and by x
+// through L2: three steps' loads are in flight and none past the last step is made
+// (those loads alone were 5 of 12 us at M = 16). [2048, 1536] at M = 12 takes 5.8 us,
+// gate + up [6144, 1536] 9.8, [1536, 6144] 14.7 (7.2, 19.0 and 19.3 as words).
+template <int BITS, int MODE, int RB>
+__device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
+    constexpr int NWT = MODE == 1 ? 2 : 1;
+    constexpr int NR = NWT * RB;  // 16-row blocks
+    constexpr int D = 3;          // steps in flight
+    constexpr int NW = 8;         // waves
+    __shared__ float red[NW][NR][4][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, rl = lane & 15;
+    const uint32_t nsteps = p.K / 64, n0 = blockIdx.x * 16 * RB;
+    const uint8_t* wp[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+        wp[q] = (q >= RB ? p.wb2 : p.wb) + (size_t)min(n0 + 16 * (q % RB) + rl, p.N - 1) * p.row_bytes + g * 2 * BITS;
+    const float* const xp = p.x + (size_t)min((uint32_t)rl, p.M - 1) * p.K + 4 * g;
+    struct Step {
+        uint32_t w[NR][BITS / 2];
+        float4 x[4];
+    };
+    auto load = [&](Step& s, uint32_t st) {
+        if (st >= nsteps) return;  // (the step index is the wave's: no divergence)
+#pragma unroll
+        for (int q = 0; q < NR; ++q) mm_load_w16<BITS>(wp[q] + (size_t)st * 8 * BITS, s.w[q]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s.x[i] = *reinterpret_cast<const float4*>(xp + (size_t)st * 64 + 16 * i);
+    };
+    typedef float f4v_ __attribute__((ext_vector_type(4)));
+    float tot[NR][4];
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tot[q][v] = 0.0f;
+    auto compute = [&](const Step& s) {
+        float x[16], mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[4 * i] = s.x[i].x;
+            x[4 * i + 1] = s.x[i].y;
+            x[4 * i + 2] = s.x[i].z;
+            x[4 * i + 3] = s.x[i].w;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(x[i]));
+        mx = g4a_col_max4(mx);  // the token's 64 k
+        const int a = max(__builtin_amdgcn_frexp_expf(mx) - 15, -126);
+        mm_h8 hi[2], lo[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float v = ldexpf(x[mm_few_x<BITS>(c, i)], -a);
+                hi[c][i] = (_Float16)v;
+                lo[c][i] = (_Float16)__builtin_fmaf((float)hi[c][i], -1.0f, v);
+            }
+        const float sc = ldexpf(1.0f, a);
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            f4v_ acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            uint32_t o[BITS == 8 ? 4 : 2];
+            mm_spread<BITS>(s.w[q], o);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const mm_h8 f = mm_few_frag<BITS>(o, i, p.xm);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(f, hi[i], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(f, lo[i], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) tot[q][v] = __builtin_fmaf(acc[v], sc, tot[q][v]);
+        }
+    };
+    Step s[D];
+#pragma unroll
+    for (int d = 0; d + 1 < D; ++d) load(s[d], w + NW * d);
+    for (uint32_t st = w; st < nsteps; st += NW * D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            load(s[(d + D - 1) % D], st + NW * (d + D - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            if (st + NW * d < nsteps) compute(s[d]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) red[w][q][v][lane] = tot[q][v];
+    __syncthreads();
+    // output (token m, row nn of the workgroup), rows next to each other across threads
+    for (uint32_t e = tid; e < 16 * 16 * RB; e += 64 * NW) {
+        const uint32_t m = e / (16 * RB), nn = e % (16 * RB), n = n0 + nn;
+        if (m >= p.M || n >= p.N) continue;
+        const int rb = nn >> 4, src = 16 * ((nn >> 2) & 3) + m;
+        float o = 0.0f, o2 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            o += red[k][rb][nn & 3][src];
+            if (MODE == 1) o2 += red[k][NR - RB + rb][nn & 3][src];
+        }
+        p.y[(size_t)m * p.N + n] = mm_out<MODE>(o * p.s[n], MODE == 1 ? o2 * p.s2[n] : 0.0f,
+                                                MODE == 2 ? p.b[(size_t)m * p.b_stride + p.b_off + n] : 0.0f);
+    }
+}
+
 }  // namespace
 
 // Forms 0 .. 3: tiles of 128 tokens x 256 / 128 rows, k-split blocks of 32 tokens x
@@ -517,11 +695,19 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
     extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_2_b##B##_mode##MODE(G4aLinearMmParams p) {      \
         linear_mm_ksplit<B, MODE, 2, 1>(p);                                                       \
     }                                                                                                             \
-    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_3_b##B##_mode##MODE(G4aLinearMmParams p) {      \
+    extern "C" __global__ __launch_bounds__(512, MODE == 1 ? 2 : 4) void g4a_linear_mm_3_b##B##_mode##MODE(         \
+        G4aLinearMmParams p) {                                                                                    \
         linear_mm_ksplit<B, MODE, 1, 1>(p);                                                                       \
+    }
+#define G4A_MM_FEW(B, MODE, RB)                                                                                   \
+    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_few_r##RB##_b##B##_mode##MODE(              \
+        G4aLinearMmParams p) {                                                                                    \
+        linear_mm_few<B, MODE, RB>(p);                                                                            \
     }
 #define G4A_MM_SET(B)                                                                                             \
     G4A_MM(B, 0) G4A_MM(B, 1) G4A_MM(B, 2)                                                                        \
+    G4A_MM_FEW(B, 0, 1) G4A_MM_FEW(B, 0, 2) G4A_MM_FEW(B, 1, 1) G4A_MM_FEW(B, 1, 2) G4A_MM_FEW(B, 2, 1)             \
+    G4A_MM_FEW(B, 2, 2)                                                                                           \
     extern "C" __global__ __launch_bounds__(256) void g4a_split_x_b##B(G4aSplitXParams p) { split_x<B>(p); }
 G4A_MM_SET(2)
 G4A_MM_SET(4)

@@ -1,5 +1,6 @@
-"""Projections of 16 and more rows on split activations (linear_mm_*): every form
-(128-token tiles of 256 and 128 rows, 32-token k-split blocks of 64 and 32 rows)
+"""Projections of 2 and more rows on split activations (linear_mm_*): every form
+(128-token tiles of 256 and 128 rows, 32-token k-split blocks of 64 and 32 rows,
+16-token blocks of 32 and 16), the int8 kernel over pairs of rows of a large weight,
 at ragged edges of its tiles and steps, every weight format and epilogue, against
 the CPU oracle within the bound of another f32 summation order
 (2e-6 * sum |x w| + 1e-7 per output, as tests/test_linear_gpu.py derives it);
@@ -29,6 +30,16 @@ pytestmark = pytest.mark.gpu
     ("geglu", 3100, 320, 700, 2, False),
     ("geglu", 1050, 320, 900, 8, True),
     ("gelu_cols", 4099, 320, 600, 4, False),
+    ("linear", 33, 64, 2, 4, False),         # 2 .. 16 rows: x split in registers, fewer steps than waves
+    ("linear", 2050, 1600, 16, 2, False),
+    ("linear", 100, 1536, 7, 8, True),
+    ("linear", 17, 6144, 15, 8, False),
+    ("geglu", 100, 448, 3, 4, False),
+    ("geglu", 8200, 576, 13, 2, False),
+    ("geglu", 45, 1600, 5, 8, True),
+    ("gelu_cols", 95, 1600, 12, 4, False),
+    ("linear", 16400, 320, 9, 4, False),
+    ("linear", 16400, 320, 3, 2, False),
 ])
 def test_forms_match_the_oracle(ctx, op, N, K, M, bits, signed):
     name = f"{op} N={N} K={K} M={M} b{bits}{'s' if signed else ''}"
@@ -64,7 +75,7 @@ def test_weights_at_eight_byte_alignment(ctx, bits, signed):
     raw.free()
 
 
-@pytest.mark.parametrize("M", [20, 400])
+@pytest.mark.parametrize("M", [9, 20, 400])
 def test_scales_apart_and_non_finite_rows(ctx, M):
     N, K = 2048, 1024
     w, x = _qw(5, N, K, 4, False, None), synth.normal_f32(6, 1, M * K).reshape(M, K).copy()
@@ -87,6 +98,21 @@ def test_scales_apart_and_non_finite_rows(ctx, M):
     assert np.all(np.abs(got[fine].astype(np.float64) - want) <= 2e-6 * _bound(x[fine], w) + 1e-7 * unit)
     assert not got[4].any()
     assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
+
+
+@pytest.mark.parametrize("M", [3, 8, 9])
+def test_rows_of_a_large_weight(ctx, M):
+    # 64 MiB and more of packed weights: pairs of rows on the int8 matrix cores up to 8 rows
+    N, K = 131077, 2048
+    w, x = _qw(11, N, K, 2, False, None), synth.normal_f32(12, 1, M * K).reshape(M, K)
+    print(f"[gpu] M={M}", flush=True)
+    rows = np.r_[0:40, 70000:70040, N - 40:N]
+    part = oracle.QWeight(np.ascontiguousarray(w.qbytes.reshape(N, -1)[rows]), w.scales.reshape(N, -1)[rows], rows.size, K,
+                          2)
+    with Dev(ctx) as d:
+        y = d.empty((M, N))
+        ctx.linear_q(d.w(w), d.arr(x).ptr, y.ptr, M)
+        _check_sum(y.to_host()[:, rows], oracle.linear_q(x, part), _bound(x, part), f"M={M}")
 
 
 def test_capture_without_room_for_the_split(ctx):
