@@ -1243,7 +1243,7 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
     // with 64-key-multiple splits sized for one 8-wave workgroup per CU over the
     // launch's keys.
     struct Launch {
-        uint32_t first, count, kps, max_split;
+        uint32_t first, count, kps, wgs, max_split;
         bool wave, rows, wide;  // streaming kernel; combines of <= COMBINE_ROW_SPLITS / more splits
         bool kpos;              // explicit key positions
         size_t part;  // floats
@@ -1252,7 +1252,7 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
     size_t part_floats = 0;
     for (uint32_t c0 = 0; c0 < batch.size();) {
         const uint32_t c1 = c0 < n_contig ? n_contig : uint32_t(batch.size());
-        Launch L{c0, std::min<uint32_t>(G4A_BATCH_SEQ, c1 - c0), SHORT_KEYS, 0, false, false, false, c0 >= n_contig,
+        Launch L{c0, std::min<uint32_t>(G4A_BATCH_SEQ, c1 - c0), SHORT_KEYS, 0, 0, false, false, false, c0 >= n_contig,
                  part_floats};
         c0 += L.count;
         uint64_t short_wgs = 0, keys = 0;
@@ -1267,11 +1267,25 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
             L.wave = true;
             uint64_t kps = ctx->batch_kps ? ctx->batch_kps : (keys * ref->Hkv + cus - 1) / cus;
             kps = std::max<uint64_t>(kps, (max_keys + MAX_SPLITS - 1) / MAX_SPLITS);
-            L.kps = uint32_t((std::max<uint64_t>(kps, 1) + TILE - 1) / TILE * TILE);
+            if (ctx->batch_kps) {
+                L.kps = uint32_t((std::max<uint64_t>(kps, 1) + TILE - 1) / TILE * TILE);
+            } else {
+                // the fewest keys (in the kernel's 16-key tiles) with at most one workgroup per
+                // CU: the ragged sequences' last splits count as whole workgroups
+                L.kps = uint32_t((std::max<uint64_t>(kps, 1) + 15) / 16 * 16);
+                auto wgs = [&] {
+                    uint64_t n = 0;
+                    for (uint32_t j = L.first; j < L.first + L.count; ++j)
+                        n += (an[batch[j]].plan.k_end - an[batch[j]].plan.k_start + L.kps - 1) / L.kps;
+                    return n * ref->Hkv;
+                };
+                while (L.kps < max_keys && wgs() > cus) L.kps += std::max(16u, L.kps / 32 / 16 * 16);
+            }
         }
         for (uint32_t j = L.first; j < L.first + L.count; ++j) {
             const uint32_t nk = an[batch[j]].plan.k_end - an[batch[j]].plan.k_start;
             const uint32_t ns = (nk + L.kps - 1) / L.kps;
+            L.wgs += ns;
             L.max_split = std::max(L.max_split, ns);
             if (ns > 1) {
                 (ns <= COMBINE_ROW_SPLITS ? L.rows : L.wide) = true;
@@ -1297,6 +1311,8 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
         bp.softcap = ref->attn_softcap;
         bp.kpos = kpos_dev;
         size_t off = L.part;
+        uint32_t wg = 0;
+        std::fill(bp.first + L.count, bp.first + G4A_BATCH_SEQ, 0xFFFFFFFFu);
         for (uint32_t j = 0; j < L.count; ++j) {
             const g4a_attn_args& a = args[batch[L.first + j]];
             const g4a_attn_plan& pl = an[batch[L.first + j]].plan;
@@ -1318,15 +1334,19 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
                 d.kpos = G4A_NO_KPOS;
             }
             const uint32_t ns = (pl.k_end - pl.k_start + L.kps - 1) / L.kps;
+            bp.first[j] = wg;
+            wg += ns;
             d.part = uint32_t(ns > 1 ? off : 0);
             if (ns > 1) off += (size_t(ref->Hq) * ns * (ref->Dh + 2) + 63) & ~size_t(63);
         }
+        // (see decode_wave_batch for the two grids)
+        const bool one_row = L.wgs != L.max_split * L.count && (L.wave || d512);
         hipFunction_t f = L.kpos ? ctx->decode_wave_batch_kpos[d512]
                           : L.wave ? ctx->decode_wave_batch[d512] : ctx->decode_batch[d512];
-        if (int rc = launch(ctx, f, dim3(L.max_split, L.count, bp.Hkv), dim3(L.wave ? 512 : 256, 1, 1), bp,
-                            "batched decode", true))
+        if (int rc = launch(ctx, f, one_row ? dim3(L.wgs, 1, bp.Hkv) : dim3(L.max_split, L.count, bp.Hkv),
+                            dim3(L.wave ? 512 : 256, 1, 1), bp, "batched decode", true))
             return rc;
-        if (L.rows)
+        if (L.rows && !L.wide)
             if (int rc = launch(ctx, ctx->combine_rows_batch[d512], dim3(bp.Hq, L.count, 1), dim3(256, 1, 1), bp,
                                 "batched combine", true))
                 return rc;

@@ -1507,10 +1507,14 @@ __device__ __forceinline__ void combine_row_stage(const float* __restrict__ part
 }
 
 // Batched decode: one launch over the independent single-query steps of
-// b.seq[]; grid (largest split count, sequences, Hkv). The decode parameters of
-// sequence blockIdx.y are rebuilt from its descriptor (T = 1; key positions
-// relative to its first cache key, or explicit ones from b.kpos); a workgroup
-// past the sequence's split count exits at once.
+// b.seq[]. The decode parameters of a workgroup's sequence are rebuilt from its
+// descriptor (T = 1; key positions relative to its first cache key, or explicit
+// ones from b.kpos). Sequences of different split counts run on a grid of one row
+// without empty workgroups (a workgroup finds its sequence): with a (largest split
+// count, sequences) grid theirs fell unevenly on the 8 XCDs, and one with more
+// than 32 (a CU holds one) ran them in two rounds: 16 sequences of 8192 .. 512
+// keys 59 -> 40 us. Equal counts take the (splits, sequences) grid, and so does the
+// short kernel at head_dim 256, whose workgroups share CUs: the search is 0.7 us.
 __device__ __forceinline__ bool batch_params(const G4aBatchParams& b, uint32_t si, G4aDecodeParams& p) {
     const G4aSeqDesc& sd = b.seq[si];
     p = G4aDecodeParams{};
@@ -1538,36 +1542,55 @@ __device__ __forceinline__ bool batch_params(const G4aBatchParams& b, uint32_t s
     return p.nsplit > 0;
 }
 
+// This workgroup's sequence and split: (splits, sequences) grids give them, else
+// (one row) the search of `first` does, one entry per lane.
+__device__ __forceinline__ uint32_t batch_item(const G4aBatchParams& b, uint32_t& split) {
+    if (gridDim.y > 1) {
+        split = blockIdx.x;
+        return blockIdx.y;
+    }
+    const uint32_t f = b.first[threadIdx.x & 63];
+    const uint32_t si = (uint32_t)__builtin_popcountll(__ballot(f <= blockIdx.x)) - 1u;
+    split = blockIdx.x - (uint32_t)__builtin_amdgcn_readlane((int)f, (int)si);
+    return __builtin_amdgcn_readfirstlane(si);
+}
+
 template <int DH>
 __device__ __forceinline__ void decode_short_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
-    if (!batch_params(b, blockIdx.y, p) || blockIdx.x >= p.nsplit) return;
-    decode_short<DH>(p, blockIdx.x, 0u);
+    uint32_t split;
+    if (!batch_params(b, batch_item(b, split), p) || split >= p.nsplit) return;
+    decode_short<DH>(p, split, 0u);
 }
 
 template <int DH, bool KPOS>
 __device__ __forceinline__ void decode_wave_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
-    if (!batch_params(b, blockIdx.y, p) || blockIdx.x >= p.nsplit) return;
-    decode_wave<DH, KPOS>(p, blockIdx.x, 0u);
+    uint32_t split;
+    if (!batch_params(b, batch_item(b, split), p) || split >= p.nsplit) return;
+    decode_wave<DH, KPOS>(p, split, 0u);
 }
 
 // The LSE combines of a batched decode, each sequence merged by the kernel a
 // single call with its split count uses: more than COMBINE_ROW_SPLITS splits
-// here, grid (DH/COMBINE_DIMS, Hq, sequences) of COMBINE_THREADS ...
+// over DH/COMBINE_DIMS blocks of COMBINE_THREADS per head; 2 .. COMBINE_ROW_SPLITS
+// by the first 256 threads of a head's first block. One launch, grid
+// (DH/COMBINE_DIMS, Hq, sequences), for both (a launch each took 5 us more).
 template <int DH>
 __device__ __forceinline__ void combine_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
-    if (!batch_params(b, blockIdx.z, p) || p.nsplit <= COMBINE_ROW_SPLITS) return;
+    if (!batch_params(b, blockIdx.z, p) || p.nsplit < 2) return;
     const G4aCombineParams cp{p.part, p.out, 1u, b.Hq, p.nsplit, (uint32_t)DH};
-    combine<DH>(cp, 0u);
+    if (p.nsplit > COMBINE_ROW_SPLITS) combine<DH>(cp, 0u);
+    else if (blockIdx.x == 0 && threadIdx.x < 256) combine_rows<DH>(cp, blockIdx.y, 0u);
 }
 
-// ... and 2 .. COMBINE_ROW_SPLITS splits here, grid (Hq, sequences).
+// The same for a launch whose sequences all have at most COMBINE_ROW_SPLITS
+// splits: grid (Hq, sequences) of 256 threads.
 template <int DH>
 __device__ __forceinline__ void combine_rows_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
-    if (!batch_params(b, blockIdx.y, p) || p.nsplit < 2 || p.nsplit > COMBINE_ROW_SPLITS) return;
+    if (!batch_params(b, blockIdx.y, p) || p.nsplit < 2) return;
     const G4aCombineParams cp{p.part, p.out, 1u, b.Hq, p.nsplit, (uint32_t)DH};
     combine_rows<DH>(cp, blockIdx.x, 0u);
 }

@@ -337,3 +337,30 @@ def test_explicit_key_positions_batch(ctx):
             assert_parity(s.out.to_host(), s.want(), f"explicit hd512 S={s.S}")
     finally:
         _free(seqs)
+
+
+@pytest.mark.parametrize("Dh,window,lens", [
+    (512, 0, [8192, 4097, 300, 31, 5000, 1, 77]),        # streaming kernel, one row of workgroups
+    (512, 0, [300, 33, 32, 1, 64, 257]),                 # short kernel, one row
+    (512, 0, [2048, 2048, 2048, 2048]),                  # equal split counts: (splits, sequences)
+    (256, 512, [700, 3, 512, 100]),                      # head_dim 256, short kernel
+    (256, 512, [600, 40, 512, 9, 800, 511, 120] * 9),    # 63 sequences, streaming kernel
+])
+def test_ragged_batches_match_single_steps(ctx, Dh, window, lens):
+    # each sequence against the oracle, for both grids of both kernels and combines of few and
+    # many splits in one launch
+    print(f"[gpu] Dh={Dh} lens={lens[:7]} x {len(lens)}", flush=True)
+    ins = [synth.gemma_inputs(T=1, S=S, Dh=Dh, seed=900 + i) for i, S in enumerate(lens)]
+    bufs = [[ctx.upload(x) for x in (c.q, c.k, c.v)] + [ctx.empty((1, 8 * Dh))] for c in ins]
+    try:
+        calls = [dict(q=b[0].ptr, k=b[1].ptr, v=b[2].ptr, out=b[3].ptr, T=1, S=S, Hq=8, Hkv=1, Dh=Dh, Dv=Dh,
+                      q_pos0=S - 1, window=window) for b, S in zip(bufs, lens)]
+        assert ctx.attention_decode_batch(calls) == len(lens)
+        for i, (c, b) in enumerate(zip(ins, bufs)):
+            want = oracle.attention(c.q, c.k, c.v, c.q_pos, c.k_pos, window=window)
+            d = np.abs(b[3].to_host().astype(np.float64) - want)
+            assert d.max() <= 1e-5 and d.mean() <= 1e-6, f"sequence {i} ({lens[i]} keys): {d.max():.2e} {d.mean():.2e}"
+    finally:
+        for b in bufs:
+            for x in b:
+                x.free()
