@@ -130,7 +130,7 @@ struct g4a_ctx {
     hipFunction_t linear_words[3][3][3] = {};  // [bits 2/4/8][(MT, RU) = (1, 2), (1, 8), (4, 4)][mode]
     hipFunction_t linear_elem[3] = {};         // [mode]
     hipFunction_t linear_mfma[3][2][3] = {};   // [bits 2/4/8][64 / 128 weight rows per tile][mode]: M >= 16
-    hipFunction_t linear_mm[4][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
+    hipFunction_t linear_mm[5][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
     hipFunction_t linear_few[2][3][3] = {};    // [16 / 64 rows a workgroup][bits][mode]: at most 16 activation rows
     hipFunction_t split_x[3] = {};             // [bits 2/4/8]: the split
     hipFunction_t linear_i8[3][2] = {};        // [bits 2/4/8][M = 1, 2]: int8 matrix cores, mode 0
@@ -762,7 +762,7 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
                     snprintf(name, sizeof name, "g4a_linear_mm_few_r%d_b%d_mode%d", r ? 2 : 1, bits[b], m);
                     if (int rc = get_fn(ctx, &ctx->linear_few[r][b][m], name)) return bail(rc);
                 }
-                for (int f = 0; f < 4; ++f) {
+                for (int f = 0; f < 5; ++f) {
                     snprintf(name, sizeof name, "g4a_linear_mm_%d_b%d_mode%d", f, bits[b], m);
                     if (int rc = get_fn(ctx, &ctx->linear_mm[f][b][m], name)) return bail(rc);
                 }
@@ -1667,22 +1667,27 @@ LinearChoice choose_linear(const g4a_ctx* ctx, int mode, const g4a_qweight* w, c
     return c;
 }
 
-// The linear_mm form of a call: the one whose workgroups take the least time,
-// ceil(workgroups / CUs) of them after one another on a CU, at `step` us per 64 k
-// and `fixed` us per workgroup (measured with every CU busy, 4-bit; 8-bit weights'
-// loads take the k-split forms and the one-wave-a-SIMD tile longer). The choice is
-// within 10 % of the best form over M = 16 .. 2048 of [2048, 1536], [1536, 6144],
-// [1536, 12288] and gate + up [6144, 1536], [12288, 1536] weights at 2, 4 and 8 bits.
+// The linear_mm form of a call: the one whose workgroups take the least time. A
+// form's r = ceil(workgroups / CUs) workgroups per CU take r * (step us per 64 k +
+// fixed us), or for r = 1, with the CU to itself, solo (measured with every CU busy,
+// 4-bit; 8-bit weights take `wide` times as long). Against every form at M = 64 ..
+// 2048 of [2048, 1536], [1536, 6144], [1536, 12288] and gate + up [6144, 1536],
+// [12288, 1536] weights at 2, 4 and 8 bits, the choice is within 10 % of the best.
 struct MmForm {
     int form;
     uint32_t rows, toks, threads;  // weight rows (of each weight) and tokens of a workgroup
-    float step[2], fixed, wide;    // mode 0 and 2, mode 1; factor at 8 bits
+    bool tile;                     // holds rows of both weights in mode 1; copies weights 16 bytes at a time
+    struct {
+        float step, fixed;
+    } each[2], solo[2];            // modes 0 and 2, mode 1
+    float wide;
 };
-constexpr MmForm MM_FORMS[4] = {
-    {0, 256, 128, 512, {1.85f, 1.85f}, 4.0f, 1.0f},
-    {1, 128, 128, 256, {1.05f, 1.05f}, 4.0f, 1.45f},
-    {2, 64, 32, 512, {0.19f, 0.33f}, 2.0f, 1.7f},
-    {3, 32, 32, 512, {0.131f, 0.18f}, 1.1f, 1.4f},
+constexpr MmForm MM_FORMS[5] = {
+    {0, 256, 128, 512, true, {{1.75f, 4.0f}, {1.75f, 4.0f}}, {{1.35f, 8.0f}, {1.35f, 8.0f}}, 1.0f},
+    {1, 128, 128, 256, true, {{0.95f, 3.5f}, {0.95f, 3.5f}}, {{1.1f, 6.0f}, {1.1f, 6.0f}}, 1.3f},
+    {2, 64, 32, 512, false, {{0.19f, 2.0f}, {0.33f, 2.0f}}, {{0.2f, 3.0f}, {0.33f, 3.0f}}, 1.7f},
+    {3, 32, 32, 512, false, {{0.131f, 1.1f}, {0.18f, 1.1f}}, {{0.115f, 2.5f}, {0.2f, 2.4f}}, 1.4f},
+    {4, 128, 64, 256, true, {{0.5f, 1.5f}, {0.5f, 1.5f}}, {{0.72f, 6.0f}, {0.72f, 6.0f}}, 1.1f},
 };
 
 MmForm linear_mm_choose(const g4a_ctx* ctx, int mode, int bi, uint32_t M, uint32_t N, uint32_t K, bool tiles) {
@@ -1690,11 +1695,12 @@ MmForm linear_mm_choose(const g4a_ctx* ctx, int mode, int bi, uint32_t M, uint32
     MmForm best = MM_FORMS[3];
     float least = 3.0e38f;
     for (MmForm f : MM_FORMS) {
-        if (f.form <= 1 && !tiles) continue;
-        if (mode == 1 && f.form <= 1) f.rows /= 2;  // the tiles hold rows of both weights
+        if (f.tile && !tiles) continue;
+        if (mode == 1 && f.tile) f.rows /= 2;
         const uint64_t wgs = uint64_t((N + f.rows - 1) / f.rows) * ((M + f.toks - 1) / f.toks);
-        const float t = float((wgs + cus - 1) / cus) *
-                        (f.step[mode == 1] * (bi == 2 ? f.wide : 1.0f) * float(K / 64) + f.fixed);
+        const uint64_t r = (wgs + cus - 1) / cus;
+        const auto& c = (r == 1 ? f.solo : f.each)[mode == 1];
+        const float t = float(r) * (c.step * float(K / 64) + c.fixed) * (bi == 2 ? f.wide : 1.0f);
         if (t < least) least = t, best = f;
     }
     return best;

@@ -191,80 +191,90 @@ __device__ __forceinline__ void mm_store(const G4aLinearMmParams& p, const float
     }
 }
 
-// 4 bytes per lane straight to LDS (lane i at dst + i); see copy16_to_lds.
-__device__ __forceinline__ void copy4_to_lds(const void* src, float* lds_dst) {
+// 4 bytes per lane straight to LDS (lane i at dst + i); see copy16s_to_lds.
+__device__ __forceinline__ void copy4s_to_lds(const void* sbase, uint32_t voff, float* lds_dst) {
     const uint32_t m0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) float*)lds_dst);
-    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "{m0}"(m0) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
 }
 
-// Many rows: workgroup = 128 tokens x 32 NW weight rows (mode 1: half of them of
-// each weight), NW waves of 64 x 64. Per 64-k step the split x tile (32 KiB), the
-// packed weights and the scales stream into a 2-slot LDS ring by global->LDS
-// copies: once every wave holds a step's last operands in registers (at its third
-// of four MFMA steps) its slot takes the step after next. A wave issues 32 MFMAs
-// (1024 cycles) per step with one operand set being read and unpacked ahead of
-// them; with the reads placed where used, a step took 1.3 us instead of 0.85
-// (4 waves, one workgroup). With every CU busy the matrix pipe is busy half the
-// cycles, and the clock falls from 2.4 to 1.8 GHz: gate + up 4-bit [6144, 1536] at
-// M = 2048 takes 155 us (1000 TFLOP/s of fp16 products), 235 with three bf16 parts.
-template <int BITS, int MODE, int NW>
+// Many rows: workgroup = 64 TB tokens x 32 NW weight rows (mode 1: half of them of
+// each weight), NW waves of 64 rows x 32 TB tokens. Per 64-k step the split x tile (8
+// KiB per token block), the packed weights and the scales stream into a 2-slot LDS
+// ring by global->LDS copies: once every wave holds a step's last operands in
+// registers (at its third of four MFMA steps) its slot takes the step after next. At
+// TB = 2 a wave issues 32 MFMAs (1024 cycles) per step with one operand set being read
+// and unpacked ahead of them; with the reads placed where used, a step took 1.3 us
+// instead of 0.8 (4 waves, one workgroup). Bound by the MFMAs and the vector
+// instructions between them, which do not overlap: with every CU busy the matrix pipe
+// works half the cycles, and the clock falls from 2.4 to 1.8 GHz. Gate + up 4-bit
+// [6144, 1536] at M = 2048 takes 154 us (1000 TFLOP/s of fp16 products), 235 with three
+// bf16 parts; 161 with 64-bit copy addresses per lane and the sums cleared after a fold.
+template <int BITS, int MODE, int NW, int TB>
 __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
-    constexpr int CX = 32 / NW;                  // x copies per wave and step
+    constexpr int XF = 4096 * TB;                // floats of a step's x tile (2 TB token blocks)
+    constexpr int CX = 16 * TB / NW;             // x copies per wave and step
     constexpr int CW = BITS == 4 ? 1 : 2;        // weight copies (4 bytes a lane at 2 bits, else 16)
     constexpr int WL = BITS == 2 ? 64 : 256;     // floats per weight copy
     constexpr int NV = CX + CW + 1;              // copies per step
-    constexpr int SLOT = 8192 + NW * CW * WL + 128;
+    constexpr int SLOT = XF + NW * CW * WL + 64 * TB;
     __shared__ __attribute__((aligned(16))) float lds[2][SLOT];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = w >> 1, wt = w & 1, h = lane >> 5, rl = lane & 31;
-    const uint32_t nblk = (p.M + 31) / 32, tb0 = blockIdx.y * 4;
+    const uint32_t nblk = (p.M + 31) / 32, tb0 = blockIdx.y * 2 * TB;
     const uint32_t nsteps = p.K / 64, nseg = (p.K + MM_SEG - 1) / MM_SEG;
     const uint32_t n0 = blockIdx.x * (MODE == 1 ? 16 : 32) * NW;
     // row block b of the workgroup's NW (wave row r holds blocks 2r, 2r + 1): mode 1
     // alternates the two weights
     auto block_row = [&](int b) { return MODE == 1 ? n0 + 32 * (b >> 1) : n0 + 32 * b; };
-    const uint8_t* const wsrc = (MODE == 1 && (w & 1) ? p.wb2 : p.wb) +
-                                (size_t)min(block_row(w) + rl, p.N - 1) * p.row_bytes + h * 4 * BITS;
-    // x copy i of this wave: 1 KiB piece w * CX + i of the step's four 8 KiB token blocks
-    constexpr int WPB = NW / 4;  // waves per token block
+    // every copy is addressed as a scalar base, which the step moves, plus a lane offset
+    // (64-bit lane addresses were a fifth of the loop's vector instructions, and those do
+    // not run beside the MFMAs)
+    const uint32_t wrow = min(block_row(w), p.N - 1);  // a block past N re-reads the last row
+    const uint8_t* const wsrc = (MODE == 1 && (w & 1) ? p.wb2 : p.wb) + (size_t)wrow * p.row_bytes;
+    const uint32_t woff = min((uint32_t)rl, p.N - 1 - wrow) * p.row_bytes + h * 4 * BITS;
+    // x copy i of this wave: 1 KiB piece w * CX + i of the step's 8 KiB token blocks
+    constexpr int WPB = NW / (2 * TB);  // waves per token block
     const float* const xsrc = reinterpret_cast<const float*>(p.xs) +
-                              (size_t)min(tb0 + w / WPB, nblk - 1) * p.K * 32 + (w % WPB) * CX * 256 + 4 * lane;
-    // scales of token blocks 2 (w % 2) + h
-    const float* const ssrc = p.xscale + (size_t)min(tb0 + 2 * (w & 1) + h, nblk - 1) * nseg * 32 + rl;
+                              (size_t)min(tb0 + w / WPB, nblk - 1) * p.K * 32 + (w % WPB) * CX * 256;
+    const uint32_t xoff = 16 * lane;
+    // scales of two token blocks (at TB = 2 of this wave's two)
+    const uint32_t sb = min(tb0 + (TB == 2 ? 2 * (w & 1) : 0), nblk - 1);
+    const float* const ssrc = p.xscale + (size_t)sb * nseg * 32;
+    const uint32_t soff = 4 * (min((uint32_t)h, nblk - 1 - sb) * nseg * 32 + rl);
     // copy c (< NV) of step st
     auto issue_one = [&](uint32_t st, float* d, int c) {
         if (c < CX) {
-            copy16_to_lds(xsrc + (size_t)st * 2048 + 256 * c, d + 256 * (w * CX + c));
+            copy16s_to_lds(xsrc + (size_t)st * 2048 + 256 * c, xoff, d + 256 * (w * CX + c));
         } else if (c < CX + CW) {
             const int j = c - CX;
-            float* const wd = d + 8192 + (w * CW + j) * WL;
+            float* const wd = d + XF + (w * CW + j) * WL;
             const uint8_t* src = wsrc + (size_t)st * 8 * BITS;
-            if constexpr (BITS == 2) copy4_to_lds(src + 4 * j, wd);
-            else copy16_to_lds(reinterpret_cast<const float*>(src + 16 * j), wd);
+            if constexpr (BITS == 2) copy4s_to_lds(src + 4 * j, woff, wd);
+            else copy16s_to_lds(src + 16 * j, woff, wd);
         } else {
-            copy4_to_lds(ssrc + (st >> 2) * 32, d + 8192 + NW * CW * WL + 64 * (w & 1));
+            copy4s_to_lds(ssrc + (st >> 2) * 32, soff, d + XF + NW * CW * WL + (TB == 2 ? 64 * (w & 1) : 0));
         }
     };
     auto issue = [&](uint32_t st, int slot) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) issue_one(st, lds[slot], c);
     };
-    mm_f16v tot[2][2], acc[2][2];
+    mm_f16v tot[2][TB], acc[2][TB];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
+        for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) tot[rb][tb][v] = acc[rb][tb][v] = 0.0f;
+            for (int v = 0; v < 16; ++v) tot[rb][tb][v] = 0.0f;
     uint32_t wc[2][BITS];
-    mm_h8 a[2][2], bx[2][2][2];  // operands of two MFMA steps: [step & 1][row block], [step & 1][part][token block]
+    mm_h8 a[2][2], bx[2][2][TB];  // operands of two MFMA steps: [step & 1][row block], [step & 1][part][token block]
     auto read_w = [&](const float* d) {
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
             for (int j = 0; j < CW; ++j) {
-                const float* const ws = d + 8192 + ((2 * wr + rb) * CW + j) * WL;
+                const float* const ws = d + XF + ((2 * wr + rb) * CW + j) * WL;
                 if constexpr (BITS == 2) {
                     wc[rb][j] = reinterpret_cast<const uint32_t*>(ws)[lane];
                 } else {
@@ -277,20 +287,25 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
             }
     };
     auto read_x = [&](const float* d, int i) {
-        const float* const xb = d + 4096 * wt + 1024 * h + 4 * rl;
+        const float* const xb = d + 2048 * TB * wt + 1024 * h + 4 * rl;
 #pragma unroll
         for (int part = 0; part < 2; ++part)
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+            for (int tb = 0; tb < TB; ++tb)
                 bx[i & 1][part][tb] = *reinterpret_cast<const mm_h8*>(xb + 2048 * tb + (2 * i + part) * 128);
     };
     auto unpack_w = [&](int i) {
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb) a[i & 1][rb] = mm_frag<BITS>(wc[rb], i, p.xm);
     };
-    auto mfma = [&](int i, int n) {  // the n-th of step i's 8
-        const int part = n >> 2, tb = (n >> 1) & 1, rb = n & 1;
-        acc[rb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i & 1][rb], bx[i & 1][part][tb], acc[rb][tb], 0, 0, 0);
+    auto mfma = [&](int i, int n, bool zero) {  // the n-th of step i's 4 TB; zero: onto 0
+        const int part = n / (2 * TB), tb = (n >> 1) % TB, rb = n & 1;
+        mm_f16v c = acc[rb][tb];
+        if (zero) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+        }
+        acc[rb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i & 1][rb], bx[i & 1][part][tb], c, 0, 0, 0);
     };
     issue(0, 0);
     if (nsteps > 1) issue(1, 1);
@@ -300,64 +315,63 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
     read_w(lds[0]);
     read_x(lds[0], 0);
     unpack_w(0);
-    for (uint32_t st = 0; st < nsteps; ++st) {
-        float* const d = lds[st & 1];
-        const float* const dn = lds[(st & 1) ^ 1];
-        const bool fold = (st & 3) == 3 || st + 1 == nsteps;  // the segment ends here
-        float sc[2] = {0.0f, 0.0f};
-        if (fold) {
+    for (uint32_t st0 = 0; st0 < nsteps; st0 += 4) {  // a segment of x's scales
+        float sc[TB];
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) sc[tb] = d[8192 + NW * CW * WL + 64 * wt + 32 * tb + rl];
-        }
-        // operands come one MFMA step ahead, their LDS reads and unpacking spread over
-        // the MFMAs in flight
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t st = st0 + u;
+            if (u > 0 && st >= nsteps) break;
+            float* const d = lds[u & 1];
+            const float* const dn = lds[(u & 1) ^ 1];
+            if (u == 0) {
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            read_x(d, i + 1);
-            unpack_w(i + 1);
+                for (int tb = 0; tb < TB; ++tb) sc[tb] = d[XF + NW * CW * WL + 32 * (TB * wt + tb) + rl];
+            }
+            // operands come one MFMA step ahead, their LDS reads and unpacking spread over
+            // the MFMAs in flight
 #pragma unroll
-            for (int n = 0; n < 8; ++n) mfma(i, n);
+            for (int i = 0; i < 3; ++i) {
+                read_x(d, i + 1);
+                unpack_w(i + 1);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // an MFMA
-                if (j < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);             // vector ALU
+                for (int n = 0; n < 4 * TB; ++n) mfma(i, n, u == 0 && i == 0 && n < 2 * TB);
+#pragma unroll
+                for (int j = 0; j < 4 * TB; ++j) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // an MFMA
+                    if (j < 2 * TB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+                    __builtin_amdgcn_sched_group_barrier(0x002, 8 / TB, 0);             // vector ALU
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (st + 1 < nsteps) {
+                wait_vm<0>();   // step st + 1's copies, issued a step ago
+                barrier_lds();  // every wave's; every wave has read slot u & 1 for the last time
+                read_w(dn);
+                read_x(dn, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if (st + 1 < nsteps) {
-            wait_vm<0>();   // step st + 1's copies, issued a step ago
-            barrier_lds();  // every wave's; every wave has read slot st & 1 for the last time
-            read_w(dn);
-            read_x(dn, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            mfma(3, n);
-            __builtin_amdgcn_sched_barrier(0);
-            if (st + 2 < nsteps) {
+            for (int n = 0; n < 4 * TB; ++n) {
+                mfma(3, n, false);
+                __builtin_amdgcn_sched_barrier(0);
+                if (st + 2 < nsteps) {
 #pragma unroll
-                for (int c = n; c < NV; c += 8) issue_one(st + 2, d, c);
+                    for (int c = n; c < NV; c += 4 * TB) issue_one(st + 2, d, c);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if (st + 1 < nsteps) unpack_w(0);
         }
-        if (st + 1 < nsteps) unpack_w(0);
-        if (fold) {
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb)
+        for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb)
+            for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        tot[rb][tb][v] = __builtin_fmaf(acc[rb][tb][v], sc[tb], tot[rb][tb][v]);
-                        acc[rb][tb][v] = 0.0f;
-                    }
-        }
+                for (int v = 0; v < 16; ++v) tot[rb][tb][v] = __builtin_fmaf(acc[rb][tb][v], sc[tb], tot[rb][tb][v]);
     }
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb) {
-        const uint32_t m = (tb0 + 2 * wt + tb) * 32 + rl;
+    for (int tb = 0; tb < TB; ++tb) {
+        const uint32_t m = (tb0 + TB * wt + tb) * 32 + rl;
         float a[2][16];
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
@@ -682,15 +696,15 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
 
 }  // namespace
 
-// Forms 0 .. 3: tiles of 128 tokens x 256 / 128 rows, k-split blocks of 32 tokens x
-// 64 / 32 rows (in mode 1 the tiles share their rows between the weights, the blocks
-// hold as many of each).
+// Forms 0, 1, 4: tiles of 128 tokens x 256 / 128 rows and 64 tokens x 128 rows; 2, 3:
+// k-split blocks of 32 tokens x 64 / 32 rows (in mode 1 the tiles share their rows
+// between the weights, the blocks hold as many of each).
 #define G4A_MM(B, MODE)                                                                                           \
     extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_0_b##B##_mode##MODE(G4aLinearMmParams p) {      \
-        linear_mm_tile<B, MODE, 8>(p);                                                                            \
+        linear_mm_tile<B, MODE, 8, 2>(p);                                                                            \
     }                                                                                                             \
     extern "C" __global__ __launch_bounds__(256, 2) void g4a_linear_mm_1_b##B##_mode##MODE(G4aLinearMmParams p) {      \
-        linear_mm_tile<B, MODE, 4>(p);                                                                            \
+        linear_mm_tile<B, MODE, 4, 2>(p);                                                                            \
     }                                                                                                             \
     extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_2_b##B##_mode##MODE(G4aLinearMmParams p) {      \
         linear_mm_ksplit<B, MODE, 2, 1>(p);                                                       \
@@ -699,13 +713,17 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
         G4aLinearMmParams p) {                                                                                    \
         linear_mm_ksplit<B, MODE, 1, 1>(p);                                                                       \
     }
+#define G4A_MM_T64(B, MODE)                                                                                       \
+    extern "C" __global__ __launch_bounds__(256, 3) void g4a_linear_mm_4_b##B##_mode##MODE(G4aLinearMmParams p) {   \
+        linear_mm_tile<B, MODE, 4, 1>(p);                                                                         \
+    }
 #define G4A_MM_FEW(B, MODE, RB)                                                                                   \
     extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_few_r##RB##_b##B##_mode##MODE(              \
         G4aLinearMmParams p) {                                                                                    \
         linear_mm_few<B, MODE, RB>(p);                                                                            \
     }
 #define G4A_MM_SET(B)                                                                                             \
-    G4A_MM(B, 0) G4A_MM(B, 1) G4A_MM(B, 2)                                                                        \
+    G4A_MM(B, 0) G4A_MM(B, 1) G4A_MM(B, 2) G4A_MM_T64(B, 0) G4A_MM_T64(B, 1) G4A_MM_T64(B, 2)                       \
     G4A_MM_FEW(B, 0, 1) G4A_MM_FEW(B, 0, 2) G4A_MM_FEW(B, 1, 1) G4A_MM_FEW(B, 1, 2) G4A_MM_FEW(B, 2, 1)             \
     G4A_MM_FEW(B, 2, 2)                                                                                           \
     extern "C" __global__ __launch_bounds__(256) void g4a_split_x_b##B(G4aSplitXParams p) { split_x<B>(p); }

@@ -1,5 +1,5 @@
 """Projections of 2 and more rows on split activations (linear_mm_*): every form
-(128-token tiles of 256 and 128 rows, 32-token k-split blocks of 64 and 32 rows,
+(128-token tiles of 256 and 128 rows, 64-token ones of 128, 32-token k-split blocks of 64 and 32 rows,
 16-token blocks of 32 and 16), the int8 kernel over pairs of rows of a large weight,
 at ragged edges of its tiles and steps, every weight format and epilogue, against
 the CPU oracle within the bound of another f32 summation order
@@ -30,6 +30,8 @@ pytestmark = pytest.mark.gpu
     ("geglu", 3100, 320, 700, 2, False),
     ("geglu", 1050, 320, 900, 8, True),
     ("gelu_cols", 4099, 320, 600, 4, False),
+    ("linear", 2050, 1024, 990, 4, False),   # 64-token tiles
+    ("geglu", 3000, 832, 300, 8, True),
     ("linear", 33, 64, 2, 4, False),         # 2 .. 16 rows: x split in registers, fewer steps than waves
     ("linear", 2050, 1600, 16, 2, False),
     ("linear", 100, 1536, 7, 8, True),
