@@ -32,6 +32,19 @@ __device__ __forceinline__ constexpr int mm_k(int c, int pos) {
     return 8 * c + pos;
 }
 
+// The exponent a of a segment's scale 2^a from its largest |x|: not below the f32
+// normal range (it would flush), and an infinity counts as the largest float, so
+// that the finite values beside it stay finite.
+__device__ __forceinline__ int mm_scale_exp(float mx) {
+    return max(__builtin_amdgcn_frexp_expf(fminf(mx, 3.40282347e38f)) - 15, -126);
+}
+// x = +-inf leaves lo = inf - inf: any number of the weight's sign keeps the product's
+// infinity, as in f32 (a finite lo is at most 8; an x that is NaN is NaN in hi).
+__device__ __forceinline__ mm_h8 mm_lo(mm_h8 lo) {
+    const _Float16 c = (_Float16)16.0f;
+    return __builtin_elementwise_min(lo, mm_h8{c, c, c, c, c, c, c, c});
+}
+
 // x -> xs: token block tb of 32, chunk c, part p (hi, lo), token t: 8 fp16 at
 // (((tb * K/8 + c) * 2 + p) * 32 + t) * 8, so a matrix operand is 512 contiguous
 // bytes; xscale[(tb * segments + seg) * 32 + t] = 2^a. Workgroup = (segment, token
@@ -56,8 +69,7 @@ __device__ __forceinline__ void split_x(const G4aSplitXParams& p) {
 #pragma unroll
     for (int i = 0; i < 32; ++i) mx = fmaxf(mx, fabsf(x[i]));
     mx = g4a_max8(mx);  // the token's 8 threads
-    // (a scale below the f32 normal range would flush)
-    const int a = max(__builtin_amdgcn_frexp_expf(mx) - 15, -126);
+    const int a = mm_scale_exp(mx);
     if (part == 0) p.xscale[((size_t)tb * gridDim.x + seg) * 32 + tok] = ldexpf(1.0f, a);
     if (k0 >= p.K) return;
     mm_h8* const dst = reinterpret_cast<mm_h8*>(p.xs) + ((size_t)tb * (p.K / 8) + k0 / 8) * 64 + tok;
@@ -71,7 +83,7 @@ __device__ __forceinline__ void split_x(const G4aSplitXParams& p) {
             lo[i] = (_Float16)(v - (float)hi[i]);
         }
         dst[c * 64] = hi;
-        dst[c * 64 + 32] = lo;
+        dst[c * 64 + 32] = mm_lo(lo);
     }
 }
 
@@ -636,16 +648,18 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(x[i]));
         mx = g4a_col_max4(mx);  // the token's 64 k
-        const int a = max(__builtin_amdgcn_frexp_expf(mx) - 15, -126);
+        const int a = mm_scale_exp(mx);
         mm_h8 hi[2], lo[2];
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < 2; ++c) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const float v = ldexpf(x[mm_few_x<BITS>(c, i)], -a);
                 hi[c][i] = (_Float16)v;
                 lo[c][i] = (_Float16)__builtin_fmaf((float)hi[c][i], -1.0f, v);
             }
+            lo[c] = mm_lo(lo[c]);
+        }
         const float sc = ldexpf(1.0f, a);
 #pragma unroll
         for (int q = 0; q < NR; ++q) {

@@ -100,6 +100,8 @@ def test_scales_apart_and_non_finite_rows(ctx, M):
     assert np.all(np.abs(got[fine].astype(np.float64) - want) <= 2e-6 * _bound(x[fine], w) + 1e-7 * unit)
     assert not got[4].any()
     assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
+    # the infinity of its weight's sign (NaN at a weight of 0), as f32 products give it
+    assert np.array_equal(got[5], oracle.linear_q(x[5:6], w)[0], equal_nan=True)
 
 
 @pytest.mark.parametrize("M", [3, 8, 9])
