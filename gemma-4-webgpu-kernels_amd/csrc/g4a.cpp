@@ -1020,10 +1020,18 @@ int attention_run(g4a_ctx* ctx, const g4a_attn_args* a, const Analysis& an, bool
                                     ? NOALLOC_SCRATCH_BYTES + NOALLOC_PARTIAL_BYTES - part_off
                                     : SIZE_MAX;
             const PrefillTiles tiles{a, pp.q_pos0, pp.k_pos0};
-            split = prefill_split(tiles, (a->T + 7) / 8, a->Hkv, uint64_t(std::max(ctx->cu_count, 1)), d512,
-                                  uint32_t(std::min<size_t>(room / slot_bytes, PREFILL_MAX_SLOTS)));
-            const size_t need = part_off + (noalloc ? noalloc_partial_bytes(tiles, d512)
-                                                    : split.slots * a->Hkv * slot_bytes);
+            auto choose = [&](size_t bytes) {
+                split = prefill_split(tiles, (a->T + 7) / 8, a->Hkv, uint64_t(std::max(ctx->cu_count, 1)), d512,
+                                      uint32_t(std::min<size_t>(bytes / slot_bytes, PREFILL_MAX_SLOTS)));
+                return part_off + split.slots * a->Hkv * slot_bytes;
+            };
+            size_t need = choose(room);
+            if (noalloc) {
+                need = part_off + noalloc_partial_bytes(tiles, d512);
+            } else if (ctx->capturing && need > ctx->workspace_bytes && part_off <= ctx->workspace_bytes) {
+                // a capture cannot grow the workspace: no more shares than it has room for
+                need = choose(ctx->workspace_bytes - part_off);
+            }
             void* wsp = nullptr;
             if (int rc = call_workspace(ctx, need, noalloc, &wsp)) return rc;
             char* const ws = static_cast<char*>(wsp);

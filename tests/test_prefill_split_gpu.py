@@ -46,3 +46,30 @@ def test_noalloc_split_is_bit_identical(ctx, T, S):
     finally:
         for b in bufs + outs:
             b.free()
+
+
+@pytest.mark.parametrize("Dh", [256, 512])
+def test_capture_with_room_for_the_keys_only(Dh):
+    # the workspace, grown by a projection's split of 4 Dh rows (2056 floats each), holds the key
+    # splits (8 Dh bytes a key) but no partial slot: the capture records unsplit blocks
+    T, S, M, N, K = 64, 4096, 4 * Dh, 64, 2048
+    ins = synth.gemma_inputs(T=T, S=S, Dh=Dh, seed=11)
+    want = oracle.attention(ins.q, ins.k, ins.v, ins.q_pos, ins.k_pos)
+    with g4a.Context(0) as own:
+        bufs, out = [own.upload(x) for x in (ins.q, ins.k, ins.v)], own.empty((T, 8 * Dh))
+        x, y = own.upload(np.zeros((M, K), np.float32)), own.empty((M, N))
+        qb, sc = own.upload(np.zeros((N, K // 2), np.uint8)), own.upload(np.ones(N, np.float32))
+        w = g4a.DeviceQWeight(g4a.QWeightArgs(qb.ptr, sc.ptr, N, K, 4, 0, K), None, None)
+        print(f"[gpu] Dh={Dh}", flush=True)
+        own.linear_q(w, x.ptr, y.ptr, M)
+        own.sync()
+        own.capture_begin()
+        own.attention(*(b.ptr for b in bufs), out.ptr, T=T, S=S, Hq=8, Hkv=1, Dh=Dh, Dv=Dh, q_pos0=S - T)
+        graph = own.capture_end()
+        for _ in range(2):
+            graph.launch()
+            d = np.abs(out.to_host().astype(np.float64) - want)
+            assert d.max() <= 1e-5 and d.mean() <= 1e-6
+        graph.free()
+        for b in bufs + [out, x, y, qb, sc]:
+            b.free()
