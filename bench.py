@@ -701,11 +701,11 @@ def linear_bench(ctx, op, N, K, bits, M, steps, cpu=True, graph=True):
            "timing": "us_per_call: calls back to back, replayed from a captured graph (rates from it); "
                      "kernel_dispatch_us: one event pair per dispatch issued from Python"}
     if M >= 16:
-        # 2 flops per multiply-add of the projection(s), against the dense bf16 matrix peak
-        # (the kernel issues three bf16 MFMAs per multiply-add: x split into three exact parts)
+        # 2 flops per multiply-add of the projection(s), against the dense fp16 matrix peak
+        # (the kernel issues two fp16 MFMAs per multiply-add: x split into two parts)
         fl = 2 * nw * M * N * K
         res["TFLOP_s_linear"] = fl / (us * 1e-6) / 1e12
-        res["frac_bf16_mfma_peak_x3"] = 3 * fl / (us * 1e-6) / 1e12 / 2500.0
+        res["frac_fp16_mfma_peak_x2"] = 2 * fl / (us * 1e-6) / 1e12 / 2500.0
     if cpu and M * N * K <= 2e9:
         w_o = oracle.QWeight(qb, sc, N, K, bits)
         t0 = time.perf_counter()

@@ -270,7 +270,8 @@ __device__ __forceinline__ void linear_q_words(const G4aLinearParams& p) {
 }
 
 // ---------------------------------------------------------------------------
-// Prefill projections (M >= 16) on the matrix cores: v_mfma_f32_16x16x32_bf16
+// Projections of 16 and more rows that cannot split x ahead (linear_mm.hip): K <= 256,
+// or no workspace for it, as in a capture. On the matrix cores: v_mfma_f32_16x16x32_bf16
 // with exact products. x = x0 + x1 + x2 exactly, each part a bf16 holding the
 // next 8 significant bits (rounded splits of an f32 leave at most 8 bits for
 // the last part); the quantised fields times F are small integers, exact in

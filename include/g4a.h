@@ -331,11 +331,12 @@ int g4a_linear(g4a_ctx *ctx, const float *w, uint32_t N, uint32_t K, const float
  * (group_size >= K), a 4-byte aligned qbytes, 16-byte aligned x and at most
  * 16384 activations per row once the row's words are padded to a multiple of
  * 64 run the word-parallel kernel (HBM-bound, f32 sums in another order than the
- * reference's, within f32 reordering error); with M >= 16, K % 64 == 0 and an
- * 8-byte aligned qbytes they run on the matrix cores instead (x split into two
- * fp16 parts scaled by powers of two, to 2^-24 of its value, in the context's
- * workspace; f32 accumulation, the same error bound; for K <= 256, or where the
- * workspace cannot grow, three bf16 parts and exact products). g4a_linear_q with M <= 2, one scale
+ * reference's, within f32 reordering error); with M >= 2 (long rows and tall
+ * weights: M >= 5), K % 64 == 0 and an 8-byte aligned qbytes they run on the matrix
+ * cores instead (x split into two fp16 parts scaled by powers of two, to 2^-24 of
+ * its value, from M = 16 in the context's workspace; f32 accumulation, the same
+ * error bound; M >= 16 with K <= 256, or where the workspace cannot grow: three bf16
+ * parts and exact products). g4a_linear_q with M <= 2 (8 from 64 MiB), one scale
  * per row, rows of a multiple of 128 bytes, K <= 4096 (K % 64 == 0), a 16-byte
  * aligned qbytes and at least 16 MB of packed weights (the lm_head) runs on the
  * int8 matrix cores with x cut into exact digits: within a few f32 ulps of the
