@@ -132,6 +132,7 @@ struct g4a_ctx {
     hipFunction_t linear_mfma[3][2][3] = {};   // [bits 2/4/8][64 / 128 weight rows per tile][mode]: M >= 16
     hipFunction_t linear_mm[5][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
     hipFunction_t linear_few[2][3][3] = {};    // [16 / 64 rows a workgroup][bits][mode]: at most 16 activation rows
+    hipFunction_t linear_few16[3] = {};        // [bits]: mode 0, 16 rows a workgroup of 16 waves
     hipFunction_t split_x[3] = {};             // [bits 2/4/8]: the split
     hipFunction_t linear_i8[3][2] = {};        // [bits 2/4/8][M = 1, 2]: int8 matrix cores, mode 0
     // G4A_LINEAR_I8=0 keeps M <= 2 projections off the int8 matrix-core kernel,
@@ -767,6 +768,8 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
                     if (int rc = get_fn(ctx, &ctx->linear_mm[f][b][m], name)) return bail(rc);
                 }
             }
+            snprintf(name, sizeof name, "g4a_linear_mm_few_w16_b%d_mode0", bits[b]);
+            if (int rc = get_fn(ctx, &ctx->linear_few16[b], name)) return bail(rc);
             snprintf(name, sizeof name, "g4a_split_x_b%d", bits[b]);
             if (int rc = get_fn(ctx, &ctx->split_x[b], name)) return bail(rc);
         }
@@ -1802,9 +1805,11 @@ int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qwei
                                   mode == 1 ? static_cast<const uint8_t*>(w2->qbytes) : nullptr, nullptr, nullptr, x, p.s,
                                   p.s2, p.b, p.y, M, p.N, p.K, p.row_bytes, p.b_stride, p.b_off,
                                   p.signed_i8 ? 0x80808080u : 0u};
-        const uint32_t rows = ch.wide ? 32 : 16;
-        return launch(ctx, ctx->linear_few[ch.wide][bi][mode], dim3((w->N + rows - 1) / rows, 1, 1), dim3(512, 1, 1), q,
-                      "quantised linear (few rows)", true);
+        const uint32_t rows = ch.wide ? 32 : 16, steps = w->K / 64, wgs = (w->N + rows - 1) / rows;
+        // 16 waves for rows of 16 .. 32 steps where every CU has one workgroup at most (see linear_mm_few)
+        const bool w16 = mode == 0 && !ch.wide && steps >= 16 && steps <= 32 && wgs <= uint64_t(std::max(ctx->cu_count, 1));
+        return launch(ctx, w16 ? ctx->linear_few16[bi] : ctx->linear_few[ch.wide][bi][mode], dim3(wgs, 1, 1),
+                      dim3(w16 ? 1024 : 512, 1, 1), q, "quantised linear (few rows)", true);
     }
     if (ch.kind == LinearChoice::MFMA) {
         // 64 activation rows x 128 weight rows per workgroup on the matrix cores,

@@ -597,18 +597,20 @@ __device__ __forceinline__ constexpr int mm_few_x(int i, int pos) {
 }
 
 // 16 rows of x or fewer (a serving batch's step): workgroup = 16 RB weight rows (of
-// each weight), 8 waves taking every eighth 64-k step, x split in registers by the
+// each weight), NW waves taking every NW-th 64-k step, x split in registers by the
 // wave that uses it (a launch ahead for it would cost 3 us), one scale per token and
 // step; the waves' sums added through LDS in order. Bound by latency and by x
 // through L2: three steps' loads are in flight and none past the last step is made
 // (those loads alone were 5 of 12 us at M = 16). [2048, 1536] at M = 12 takes 5.8 us,
-// gate + up [6144, 1536] 9.8, [1536, 6144] 14.7 (7.2, 19.0 and 19.3 as words).
-template <int BITS, int MODE, int RB>
+// gate + up [6144, 1536] 9.8, [1536, 6144] 14.7 (7.2, 19.0 and 19.3 as words; NW = 8).
+// NW = 16 halves the chain of a row of 16 .. 32 steps: [2048, 1536] M = 12 5.5 -> 5.1,
+// M = 2 4.4 -> 4.0, [1536, 2048] M = 4 5.2 -> 4.8. Longer rows wait for x through L2
+// instead ([1536, 4096] M = 8 8.4 against 9.0), shorter ones have no step for each wave.
+template <int BITS, int MODE, int RB, int NW>
 __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
     constexpr int NWT = MODE == 1 ? 2 : 1;
     constexpr int NR = NWT * RB;  // 16-row blocks
     constexpr int D = 3;          // steps in flight
-    constexpr int NW = 8;         // waves
     __shared__ float red[NW][NR][4][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -734,12 +736,16 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
 #define G4A_MM_FEW(B, MODE, RB)                                                                                   \
     extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_few_r##RB##_b##B##_mode##MODE(              \
         G4aLinearMmParams p) {                                                                                    \
-        linear_mm_few<B, MODE, RB>(p);                                                                            \
+        linear_mm_few<B, MODE, RB, 8>(p);                                                                         \
+    }
+#define G4A_MM_FEW16(B)                                                                                           \
+    extern "C" __global__ __launch_bounds__(1024) void g4a_linear_mm_few_w16_b##B##_mode0(G4aLinearMmParams p) {    \
+        linear_mm_few<B, 0, 1, 16>(p);                                                                            \
     }
 #define G4A_MM_SET(B)                                                                                             \
     G4A_MM(B, 0) G4A_MM(B, 1) G4A_MM(B, 2) G4A_MM_T64(B, 0) G4A_MM_T64(B, 1) G4A_MM_T64(B, 2)                       \
     G4A_MM_FEW(B, 0, 1) G4A_MM_FEW(B, 0, 2) G4A_MM_FEW(B, 1, 1) G4A_MM_FEW(B, 1, 2) G4A_MM_FEW(B, 2, 1)             \
-    G4A_MM_FEW(B, 2, 2)                                                                                           \
+    G4A_MM_FEW(B, 2, 2) G4A_MM_FEW16(B)                                                                                           \
     extern "C" __global__ __launch_bounds__(256) void g4a_split_x_b##B(G4aSplitXParams p) { split_x<B>(p); }
 G4A_MM_SET(2)
 G4A_MM_SET(4)

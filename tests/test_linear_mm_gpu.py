@@ -34,7 +34,11 @@ pytestmark = pytest.mark.gpu
     ("geglu", 3000, 832, 300, 8, True),
     ("linear", 33, 64, 2, 4, False),         # 2 .. 16 rows: x split in registers, fewer steps than waves
     ("linear", 2050, 1600, 16, 2, False),
-    ("linear", 100, 1536, 7, 8, True),
+    ("linear", 100, 1536, 7, 8, True),       # 16 waves, some with one step more; at 1024 and 2048 one and two each
+    ("linear", 33, 1024, 16, 4, False),
+    ("linear", 4090, 2048, 2, 2, False),
+    ("linear", 50, 960, 5, 4, False),        # below and above their range
+    ("linear", 50, 2112, 5, 4, False),
     ("linear", 17, 6144, 15, 8, False),
     ("geglu", 100, 448, 3, 4, False),
     ("geglu", 8200, 576, 13, 2, False),
