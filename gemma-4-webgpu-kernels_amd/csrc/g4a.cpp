@@ -175,7 +175,6 @@ struct g4a_ctx {
     hipEvent_t ev_staging = nullptr;  // last use of the pinned staging buffer
     void* workspace = nullptr;
     size_t workspace_bytes = 0;
-    size_t prev_workspace_bytes = 0;  // the size of the buffer the last growth replaced
     int query_depth = 0;              // > 0 inside a query entry point (g4a_attention_plan)
     void* scratch = nullptr;  // this device's static scratch array (the allocation-free entry point)
     hipFunction_t prefill_merge[2] = {nullptr, nullptr};  // [dh512] merge of split prefill blocks
@@ -261,36 +260,64 @@ int get_fn(g4a_ctx* ctx, hipFunction_t* f, const char* name) {
     return G4A_OK;
 }
 
-int ensure_workspace(g4a_ctx* ctx, size_t bytes) {
+// Gives the workspace up: freed, or kept for the live graphs that replay with it.
+// With no graph live, those kept for earlier graphs are freed too.
+int release_workspace(g4a_ctx* ctx) {
+    std::vector<void*>& retired = ctx->book->retired;
+    if (!ctx->book->live && (ctx->workspace || !retired.empty()))
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // queued kernels may still read them
+    if (ctx->workspace) retired.push_back(ctx->workspace);
+    ctx->workspace = nullptr;
+    ctx->workspace_bytes = 0;
+    while (!ctx->book->live && !retired.empty()) {
+        void* const p = retired.back();
+        retired.pop_back();
+        HIP_TRY(ctx, hipFree(p));
+    }
+    return G4A_OK;
+}
+
+// Grows the workspace to `bytes`, by doubling where there is memory for that (a run
+// of slightly larger calls retires a bounded number of buffers). The old buffer is
+// given up once the new one is there. Where the two have no room together, a call
+// that cannot do without (`must`) gives the old one up first; any other gets
+// G4A_E_NOMEM, without a message, and the context keeps what it had. A graph capture
+// cannot grow it.
+int grow_workspace(g4a_ctx* ctx, size_t bytes, bool must) {
     if (bytes <= ctx->workspace_bytes) return G4A_OK;
-    if (ctx->capturing)
+    if (ctx->capturing) {
+        if (!must) return G4A_E_NOMEM;
         return fail(ctx, G4A_E_ARG, "the workspace must grow to %zu bytes, which a graph capture cannot do: "
                     "run the calls once before capturing them", bytes);
-    if (ctx->workspace) {
-        if (ctx->book->live) {
-            // live graphs replay with this buffer: keep it until the last one is destroyed
-            ctx->book->retired.push_back(ctx->workspace);
-        } else {
-            // the old buffer may still be read by queued kernels
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            HIP_TRY(ctx, hipFree(ctx->workspace));
+    }
+    void* grown = nullptr;
+    size_t want = std::max<size_t>({bytes, 2 * ctx->workspace_bytes, size_t(8) << 20});
+    auto allocate = [&] {
+        hipError_t e = hipMalloc(&grown, want);
+        if (e == hipErrorOutOfMemory && want > bytes) e = hipMalloc(&grown, want = bytes);
+        if (e != hipSuccess) (void)hipGetLastError();  // reported here: not to the thread's next launch check
+        return e;
+    };
+    hipError_t e = allocate();
+    if (e == hipErrorOutOfMemory && !must) return G4A_E_NOMEM;
+    if (e == hipErrorOutOfMemory) {
+        if (int rc = release_workspace(ctx)) return rc;
+        e = allocate();
+    } else if (e == hipSuccess) {
+        if (int rc = release_workspace(ctx)) {
+            (void)hipFree(grown);
+            return rc;
         }
-        ctx->prev_workspace_bytes = ctx->workspace_bytes;
-        ctx->workspace = nullptr;
-        ctx->workspace_bytes = 0;
     }
-    if (!ctx->book->live && !ctx->book->retired.empty()) {
-        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-        for (void* p : ctx->book->retired) HIP_TRY(ctx, hipFree(p));
-        ctx->book->retired.clear();
-    }
-    // geometric growth: a run of slightly larger calls retires a bounded number of buffers
-    size_t want = std::max<size_t>({bytes, 2 * ctx->prev_workspace_bytes, size_t(8) << 20});
-    hipError_t e = hipMalloc(&ctx->workspace, want);
-    if (e != hipSuccess) return fail(ctx, G4A_E_NOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
+    if (e != hipSuccess)
+        return fail(ctx, e == hipErrorOutOfMemory ? G4A_E_NOMEM : G4A_E_HIP, "workspace of %zu bytes: %s", bytes,
+                    hipGetErrorString(e));
+    ctx->workspace = grown;
     ctx->workspace_bytes = want;
     return G4A_OK;
 }
+
+int ensure_workspace(g4a_ctx* ctx, size_t bytes) { return grow_workspace(ctx, bytes, true); }
 
 // 16-key tiles of each block of 8 queries of a prefill call, as the kernels
 // count them (prefill_pair, prefill_dsplit).
@@ -1728,19 +1755,6 @@ size_t split_x_bytes(uint32_t rows, uint32_t K) {
     return size_t(rows + 31) / 32 * 32 * (size_t(K) + (K + 255) / 256) * sizeof(float);
 }
 
-// Whether the context has, or can get, the memory of a split x: not in a graph
-// capture whose workspace would grow, nor when the device is out of memory (the
-// call then takes linear_q_mfma, which needs none).
-bool linear_mm_fits(g4a_ctx* ctx, const G4aLinearParams& p) {
-    const size_t need = split_x_bytes(linear_mm_rows(p.M, p.K), p.K);
-    if (need <= ctx->workspace_bytes) return true;
-    if (ctx->capturing) return false;
-    const std::string err = ctx->err;
-    if (ensure_workspace(ctx, need) == G4A_OK) return true;
-    ctx->err = err;
-    return false;
-}
-
 int linear_mm_launch(g4a_ctx* ctx, int mode, int bi, const G4aLinearParams& p) {
     const uint32_t most = linear_mm_rows(p.M, p.K), nseg = (p.K + 255) / 256;
     for (uint32_t m0 = 0; m0 < p.M; m0 += most) {
@@ -1816,7 +1830,13 @@ int linear_q_launch(g4a_ctx* ctx, int mode, const g4a_qweight* w, const g4a_qwei
         // or x 64 rows when the larger tile would leave fewer than 2 workgroups per CU
         p.wb = static_cast<const uint8_t*>(w->qbytes);
         p.wb2 = mode == 1 ? static_cast<const uint8_t*>(w2->qbytes) : nullptr;
-        if (w->K > LINEAR_MM_MIN_K && linear_mm_fits(ctx, p)) return linear_mm_launch(ctx, mode, bi, p);
+        if (w->K > LINEAR_MM_MIN_K) {
+            // (no room for the split x, as in a graph capture whose workspace would have to
+            // grow: linear_q_mfma, which needs none)
+            const int rc = grow_workspace(ctx, split_x_bytes(linear_mm_rows(M, w->K), w->K), false);
+            if (rc == G4A_OK) return linear_mm_launch(ctx, mode, bi, p);
+            if (rc != G4A_E_NOMEM) return rc;
+        }
         const int wide = ch.wide;
         const uint32_t gx = wide ? (w->N + 127) / 128 : (w->N + 63) / 64;
         for (uint32_t m0 = 0; m0 < M; m0 += 65535u * 64) {
