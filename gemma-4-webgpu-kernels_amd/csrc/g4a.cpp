@@ -1058,9 +1058,11 @@ int attention_run(g4a_ctx* ctx, const g4a_attn_args* a, const Analysis& an, bool
             size_t need = choose(room);
             if (noalloc) {
                 need = part_off + noalloc_partial_bytes(tiles, d512);
-            } else if (ctx->capturing && need > ctx->workspace_bytes && part_off <= ctx->workspace_bytes) {
-                // a capture cannot grow the workspace: no more shares than it has room for
-                need = choose(ctx->workspace_bytes - part_off);
+            } else if (const int rc = grow_workspace(ctx, need, false)) {
+                if (rc != G4A_E_NOMEM) return rc;
+                // a capture, which cannot grow the workspace, or a device without the memory:
+                // no more shares than the workspace has room for
+                need = choose(std::max(ctx->workspace_bytes, part_off) - part_off);
             }
             void* wsp = nullptr;
             if (int rc = call_workspace(ctx, need, noalloc, &wsp)) return rc;

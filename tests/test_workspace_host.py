@@ -2,7 +2,8 @@
 for the HIP runtime: a projection of many rows takes a larger one if there is memory
 for it and else runs the kernel that needs none, with the workspace it found left
 as it was; growth by doubling does not ask for more than a tight device has; and
-errors that are not a lack of memory come back to the caller."""
+errors that are not a lack of memory come back to the caller. A prefill without
+memory for the partials of split query blocks runs them whole."""
 import pytest
 
 import hip_standin as hip
@@ -81,3 +82,21 @@ def test_errors_other_than_a_lack_of_memory_reach_the_caller(ctx):
     assert e.value.code == -1
     hip.sync_error(0)
     assert _project(ctx, 20000)[0] == "g4a_split_x_b4"
+
+
+@pytest.mark.parametrize("Dh", [256, 512])
+def test_a_prefill_with_memory_for_its_key_splits_only_runs_whole_blocks(ctx, Dh):
+    S, T = 8192, 64
+    splits = 256 + 2 * S * Dh * 4 + S // 16 * 4
+    hip.budget(hip.used() + splits + 256)
+
+    def attend():
+        ctx.attention(PTR, PTR, PTR, PTR, T=T, S=S, Hq=8, Hkv=1, Dh=Dh, Dv=Dh, q_pos0=S - T)
+        return {x.name: x.gx for x in hip.launches()}
+
+    whole = {256: "g4a_prefill2_d256", 512: "g4a_prefill2_d512"}[Dh]
+    got = attend()
+    assert got[whole] == T // 8 and len(got) == 2
+    hip.budget()
+    got = attend()
+    assert f"g4a_prefill_merge_d{Dh}" in got
