@@ -1280,8 +1280,7 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
     // (batch[0 .. n_contig)) apart from the explicit-position ones. A launch
     // whose 32-key splits fit one short-kernel workgroup per CU runs the short
     // kernel; otherwise (and always for explicit positions) the streaming kernel
-    // with 64-key-multiple splits sized for one 8-wave workgroup per CU over the
-    // launch's keys.
+    // with splits sized for one 8-wave workgroup per CU over the launch's keys.
     struct Launch {
         uint32_t first, count, kps, wgs, max_split;
         bool wave, rows, wide;  // streaming kernel; combines of <= COMBINE_ROW_SPLITS / more splits
@@ -1290,49 +1289,61 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
     };
     std::vector<Launch> launches;
     size_t part_floats = 0;
-    for (uint32_t c0 = 0; c0 < batch.size();) {
-        const uint32_t c1 = c0 < n_contig ? n_contig : uint32_t(batch.size());
-        Launch L{c0, std::min<uint32_t>(G4A_BATCH_SEQ, c1 - c0), SHORT_KEYS, 0, 0, false, false, false, c0 >= n_contig,
-                 part_floats};
-        c0 += L.count;
-        uint64_t short_wgs = 0, keys = 0;
-        uint32_t max_keys = 0;
-        for (uint32_t j = L.first; j < L.first + L.count; ++j) {
-            const uint32_t nk = an[batch[j]].plan.k_end - an[batch[j]].plan.k_start;
-            short_wgs += (nk + SHORT_KEYS - 1) / SHORT_KEYS;
-            keys += nk;
-            max_keys = std::max(max_keys, nk);
-        }
-        if (L.kpos || ctx->batch_kernel == 2 || (ctx->batch_kernel == 0 && short_wgs * ref->Hkv > cus)) {
-            L.wave = true;
-            uint64_t kps = ctx->batch_kps ? ctx->batch_kps : (keys * ref->Hkv + cus - 1) / cus;
-            kps = std::max<uint64_t>(kps, (max_keys + MAX_SPLITS - 1) / MAX_SPLITS);
-            if (ctx->batch_kps) {
-                L.kps = uint32_t((std::max<uint64_t>(kps, 1) + TILE - 1) / TILE * TILE);
-            } else {
-                // the fewest keys (in the kernel's 16-key tiles) with at most one workgroup per
-                // CU: the ragged sequences' last splits count as whole workgroups
-                L.kps = uint32_t((std::max<uint64_t>(kps, 1) + 15) / 16 * 16);
-                auto wgs = [&] {
-                    uint64_t n = 0;
-                    for (uint32_t j = L.first; j < L.first + L.count; ++j)
-                        n += (an[batch[j]].plan.k_end - an[batch[j]].plan.k_start + L.kps - 1) / L.kps;
-                    return n * ref->Hkv;
-                };
-                while (L.kps < max_keys && wgs() > cus) L.kps += std::max(16u, L.kps / 32 / 16 * 16);
+    // `by`: the keys a streaming launch's split size is a multiple of
+    auto plan = [&](uint32_t by) {
+        launches.clear();
+        part_floats = 0;
+        for (uint32_t c0 = 0; c0 < batch.size();) {
+            const uint32_t c1 = c0 < n_contig ? n_contig : uint32_t(batch.size());
+            Launch L{c0, std::min<uint32_t>(G4A_BATCH_SEQ, c1 - c0), SHORT_KEYS, 0, 0, false, false, false, c0 >= n_contig,
+                     part_floats};
+            c0 += L.count;
+            uint64_t short_wgs = 0, keys = 0;
+            uint32_t max_keys = 0;
+            for (uint32_t j = L.first; j < L.first + L.count; ++j) {
+                const uint32_t nk = an[batch[j]].plan.k_end - an[batch[j]].plan.k_start;
+                short_wgs += (nk + SHORT_KEYS - 1) / SHORT_KEYS;
+                keys += nk;
+                max_keys = std::max(max_keys, nk);
             }
-        }
-        for (uint32_t j = L.first; j < L.first + L.count; ++j) {
-            const uint32_t nk = an[batch[j]].plan.k_end - an[batch[j]].plan.k_start;
-            const uint32_t ns = (nk + L.kps - 1) / L.kps;
-            L.wgs += ns;
-            L.max_split = std::max(L.max_split, ns);
-            if (ns > 1) {
-                (ns <= COMBINE_ROW_SPLITS ? L.rows : L.wide) = true;
-                part_floats += (size_t(ref->Hq) * ns * (ref->Dh + 2) + 63) & ~size_t(63);
+            if (L.kpos || ctx->batch_kernel == 2 || (ctx->batch_kernel == 0 && short_wgs * ref->Hkv > cus)) {
+                L.wave = true;
+                uint64_t kps = ctx->batch_kps ? ctx->batch_kps : (keys * ref->Hkv + cus - 1) / cus;
+                kps = std::max<uint64_t>(kps, (max_keys + MAX_SPLITS - 1) / MAX_SPLITS);
+                L.kps = uint32_t((std::max<uint64_t>(kps, 1) + by - 1) / by * by);
+                if (by < TILE) {
+                    // the fewest keys with at most one workgroup per CU: the ragged sequences' last
+                    // splits count as whole workgroups
+                    auto wgs = [&] {
+                        uint64_t n = 0;
+                        for (uint32_t j = L.first; j < L.first + L.count; ++j)
+                            n += (an[batch[j]].plan.k_end - an[batch[j]].plan.k_start + L.kps - 1) / L.kps;
+                        return n * ref->Hkv;
+                    };
+                    while (L.kps < max_keys && wgs() > cus) L.kps += std::max(16u, L.kps / 32 / 16 * 16);
+                }
             }
+            for (uint32_t j = L.first; j < L.first + L.count; ++j) {
+                const uint32_t nk = an[batch[j]].plan.k_end - an[batch[j]].plan.k_start;
+                const uint32_t ns = (nk + L.kps - 1) / L.kps;
+                L.wgs += ns;
+                L.max_split = std::max(L.max_split, ns);
+                if (ns > 1) {
+                    (ns <= COMBINE_ROW_SPLITS ? L.rows : L.wide) = true;
+                    part_floats += (size_t(ref->Hq) * ns * (ref->Dh + 2) + 63) & ~size_t(63);
+                }
+            }
+            launches.push_back(L);
         }
-        launches.push_back(L);
+    };
+    // in the streaming kernel's 16-key tiles, or in 64 keys (fewer splits of many short
+    // sequences) as an option sets and where the workspace cannot grow to the former's partials
+    plan(ctx->batch_kps ? TILE : 16);
+    if (part_floats > 0xFFFFFFFFull) {
+        plan(TILE);
+    } else if (const int rc = grow_workspace(ctx, part_floats * sizeof(float), false)) {
+        if (rc != G4A_E_NOMEM) return rc;
+        plan(TILE);
     }
     if (part_floats > 0xFFFFFFFFull) return fail(ctx, G4A_E_SHAPE, "batched decode partials exceed 2^32 floats");
     if (part_floats)

@@ -3,7 +3,8 @@ for the HIP runtime: a projection of many rows takes a larger one if there is me
 for it and else runs the kernel that needs none, with the workspace it found left
 as it was; growth by doubling does not ask for more than a tight device has; and
 errors that are not a lack of memory come back to the caller. A prefill without
-memory for the partials of split query blocks runs them whole."""
+memory for the partials of split query blocks runs them whole, and a batch of sequences without
+room for its finer splits' partials takes fewer."""
 import pytest
 
 import hip_standin as hip
@@ -100,3 +101,25 @@ def test_a_prefill_with_memory_for_its_key_splits_only_runs_whole_blocks(ctx, Dh
     hip.budget()
     got = attend()
     assert f"g4a_prefill_merge_d{Dh}" in got
+
+
+def _batch(ctx, n, S):
+    calls = ctx.prepare_batch([dict(q=PTR, k=PTR, v=PTR, out=PTR, T=1, S=S, Hq=8, Hkv=1, Dh=512, Dv=512, q_pos0=S - 1)
+                               for _ in range(n)])
+    assert ctx.attention_decode_batch(calls) == n
+    return [(x.name, x.gx) for x in hip.launches()]
+
+
+def test_a_captured_batch_takes_the_splits_its_workspace_has_room_for(ctx):
+    # 128 sequences of 160 keys: 4 splits each (48 keys) have partials of 8.03 MiB, 3 of 64 keys 6.02
+    ctx.attention(PTR, PTR, PTR, PTR, T=1, S=1000, Hq=8, Hkv=1, Dh=512, Dv=512, q_pos0=999)  # 8 MiB of workspace
+    hip.launches()
+    ctx.capture_begin()
+    got = _batch(ctx, 128, 160)
+    ctx.capture_end().free()
+    assert got == 2 * [("g4a_decode_wave_batch_d512", 3), ("g4a_combine_rows_batch_d512", 8)]
+    # the same without memory to grow it, and eagerly
+    hip.budget(hip.used())
+    assert _batch(ctx, 128, 160) == got
+    hip.budget()
+    assert _batch(ctx, 128, 160) == 2 * [("g4a_decode_wave_batch_d512", 4), ("g4a_combine_rows_batch_d512", 8)]
