@@ -2,15 +2,19 @@
 // (gfx950), x split once ahead of them: y = x . W^T with packed 2/4/8-bit W.
 // The semantics are those of linear_q.hip (rust/src/backend_cpu.rs:174-222).
 //
-// x is cut into 32-token x 256-k segments; each token's segment is scaled by the
-// power of two that puts its largest |x| in [2^14, 2^15) and split into
-// hi = fp16(x'), lo = fp16(x' - hi): x' = hi + lo to 2^-24 of its value (2^-39 of
-// the segment's largest for the smallest). The weight fields are integers of at
-// most 8 bits, exact in fp16, so each of the two products is exact in f32 and a
-// segment's sum is one v_mfma_f32_32x32x16_f16 chain, folded into the f32 total
-// with the segment's scale by one fma. Against 64 bits that is closer than the
-// three bf16 parts of linear_q_mfma (two thirds of the accumulated terms, in
-// chains of 256 k): 6.3e-7 -> 2.0e-7 relative through a 2048-row 4-bit MLP.
+// x is cut into 32-token x 256-k segments (64 k in linear_mm_few); each token's
+// segment is scaled by the power of two that puts its largest |x| in [2^14, 2^15)
+// and split into hi = fp16(x'), lo = fp16(2^11 (x' - hi)). hi + 2^-11 lo is x' to 2^-23
+// of its value for every element within 2^-27 of the segment's largest (one f32
+// significand in four is rounded, in its last bit) and to 2^-50 of the largest for
+// smaller ones. lo's own scale is what keeps elements beside an outlier: without it
+// they are held to 2^-39 of the largest, and where the outlier meets a weight of 0 that
+// is the output's error. The weight fields are integers of at most 8 bits, exact in
+// fp16 also times 2^-11, so each product with hi or lo is exact in f32 and a segment's
+// sum is one v_mfma_f32_32x32x16_f16 chain, folded into the f32 total with the segment's
+// scale by one fma. Against 64 bits that is closer than the three bf16 parts of
+// linear_q_mfma, which hold all of x (two thirds of the accumulated terms, in chains of
+// 256 k): 6.3e-7 -> 1.8e-7 relative through a 2048-row 4-bit MLP.
 #include "g4a_math.h"
 #include "g4a_params.h"
 
@@ -20,6 +24,7 @@ typedef _Float16 mm_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 mm_h8 __attribute__((ext_vector_type(8)));
 typedef float mm_f16v __attribute__((ext_vector_type(16)));
 constexpr int MM_SEG = 256;  // k of one scale
+constexpr float MM_LO = 2048.0f;  // 2^11: lo's own scale
 
 // The order of the 8 k's of chunk c (k = 8c ..) in an operand: which k of the
 // chunk's 8 (4-, 8-bit) or of its pair's 16 (2-bit) sits at position pos. It is
@@ -38,12 +43,37 @@ __device__ __forceinline__ constexpr int mm_k(int c, int pos) {
 __device__ __forceinline__ int mm_scale_exp(float mx) {
     return max(__builtin_amdgcn_frexp_expf(fminf(mx, 3.40282347e38f)) - 15, -126);
 }
-// x = +-inf leaves lo = inf - inf: any number of the weight's sign keeps the product's
-// infinity, as in f32 (a finite lo is at most 8; an x that is NaN is NaN in hi).
-__device__ __forceinline__ mm_h8 mm_lo(mm_h8 lo) {
-    const _Float16 c = (_Float16)16.0f;
-    return __builtin_elementwise_min(lo, mm_h8{c, c, c, c, c, c, c, c});
+__device__ __forceinline__ mm_h8 mm_all(float v) {
+    const _Float16 c = (_Float16)v;
+    return mm_h8{c, c, c, c, c, c, c, c};
 }
+// x = +-inf leaves lo = inf - inf: any number of the weight's sign keeps the product's
+// infinity, as in f32 (a finite lo is at most 2^14; an x that is NaN is NaN in hi).
+__device__ __forceinline__ mm_h8 mm_lo(mm_h8 lo) { return __builtin_elementwise_min(lo, mm_all(32768.0f)); }
+__device__ __forceinline__ mm_h2 mm_pair(uint32_t v) {
+    mm_h2 r;
+    __builtin_memcpy(&r, &v, 4);
+    return r;
+}
+// The parts of eight x' = x 2^-a: hi = fp16(x'), lo = fp16(2^11 (x' - hi)). hi is converted
+// in pairs, once: the barrier keeps the compiler from converting each value again for lo.
+__device__ __forceinline__ void mm_split(const float (&x)[8], int a, mm_h8& hi, mm_h8& lo) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const mm_h2 h = {(_Float16)ldexpf(x[i], -a), (_Float16)ldexpf(x[i + 1], -a)};
+        uint32_t u;
+        __builtin_memcpy(&u, &h, 4);
+        asm("" : "+v"(u));
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            hi[i + j] = mm_pair(u)[j];
+            lo[i + j] = (_Float16)__builtin_fmaf((float)hi[i + j], -MM_LO, ldexpf(x[i + j], 11 - a));
+        }
+    }
+    lo = mm_lo(lo);
+}
+// The weight operand against lo: w / MM_LO, exact.
+__device__ __forceinline__ mm_h8 mm_frag_lo(mm_h8 w) { return w * mm_all(1.0f / MM_LO); }
 
 // x -> xs: token block tb of 32, chunk c, part p (hi, lo), token t: 8 fp16 at
 // (((tb * K/8 + c) * 2 + p) * 32 + t) * 8, so a matrix operand is 512 contiguous
@@ -76,22 +106,15 @@ __device__ __forceinline__ void split_x(const G4aSplitXParams& p) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         mm_h8 hi, lo;
+        float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float v = ldexpf(x[mm_k<BITS>(c, i)], -a);
-            hi[i] = (_Float16)v;
-            lo[i] = (_Float16)(v - (float)hi[i]);
-        }
+        for (int i = 0; i < 8; ++i) v[i] = x[mm_k<BITS>(c, i)];
+        mm_split(v, a, hi, lo);
         dst[c * 64] = hi;
-        dst[c * 64 + 32] = mm_lo(lo);
+        dst[c * 64 + 32] = lo;
     }
 }
 
-__device__ __forceinline__ mm_h2 mm_pair(uint32_t v) {
-    mm_h2 r;
-    __builtin_memcpy(&r, &v, 4);
-    return r;
-}
 // (1024 + u * 2^s) per half -> u - z: one packed fma, exact
 __device__ __forceinline__ mm_h2 mm_fix(uint32_t v, float scale, float off) {
     const mm_h2 m = {(_Float16)scale, (_Float16)scale}, o = {(_Float16)off, (_Float16)off};
@@ -228,6 +251,10 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
     constexpr int CW = BITS == 4 ? 1 : 2;        // weight copies (4 bytes a lane at 2 bits, else 16)
     constexpr int WL = BITS == 2 ? 64 : 256;     // floats per weight copy
     constexpr int NV = CX + CW + 1;              // copies per step
+    // the sums over hi and lo apart, scaled at a segment's end, or at TB = 2, which has no
+    // registers for that, weights times 2^-11 against lo: 8 packed multiplies per 8 MFMAs
+    // (gate + up of 2048 tokens 153 -> 156 us)
+    constexpr int NP = TB == 1 ? 2 : 1;
     constexpr int SLOT = XF + NW * CW * WL + 64 * TB;
     __shared__ __attribute__((aligned(16))) float lds[2][SLOT];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -272,7 +299,7 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) issue_one(st, lds[slot], c);
     };
-    mm_f16v tot[2][TB], acc[2][TB];
+    mm_f16v tot[2][TB], acc[NP][2][TB];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -280,7 +307,8 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) tot[rb][tb][v] = 0.0f;
     uint32_t wc[2][BITS];
-    mm_h8 a[2][2], bx[2][2][TB];  // operands of two MFMA steps: [step & 1][row block], [step & 1][part][token block]
+    // operands of two MFMA steps: [step & 1][row block], against lo, [step & 1][part][token block]
+    mm_h8 a[2][2], al[2], bx[2][2][TB];
     auto read_w = [&](const float* d) {
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
@@ -310,14 +338,18 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb) a[i & 1][rb] = mm_frag<BITS>(wc[rb], i, p.xm);
     };
+    auto scale_w = [&](int i, int rb) {  // step i's weights for lo
+        al[rb] = NP == 2 ? a[i & 1][rb] : mm_frag_lo(a[i & 1][rb]);
+    };
     auto mfma = [&](int i, int n, bool zero) {  // the n-th of step i's 4 TB; zero: onto 0
         const int part = n / (2 * TB), tb = (n >> 1) % TB, rb = n & 1;
-        mm_f16v c = acc[rb][tb];
+        mm_f16v& sum = acc[part % NP][rb][tb];
+        mm_f16v c = sum;
         if (zero) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) c[v] = 0.0f;
         }
-        acc[rb][tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i & 1][rb], bx[i & 1][part][tb], c, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(part ? al[rb] : a[i & 1][rb], bx[i & 1][part][tb], c, 0, 0, 0);
     };
     issue(0, 0);
     if (nsteps > 1) issue(1, 1);
@@ -346,7 +378,10 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
                 read_x(d, i + 1);
                 unpack_w(i + 1);
 #pragma unroll
-                for (int n = 0; n < 4 * TB; ++n) mfma(i, n, u == 0 && i == 0 && n < 2 * TB);
+                for (int n = 0; n < 4 * TB; ++n) {
+                    if (n < 2) scale_w(i, n);
+                    mfma(i, n, u == 0 && i == 0 && n < 2 * TB * NP);
+                }
 #pragma unroll
                 for (int j = 0; j < 4 * TB; ++j) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // an MFMA
@@ -366,6 +401,7 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
             for (int n = 0; n < 4 * TB; ++n) {
                 mfma(3, n, false);
                 __builtin_amdgcn_sched_barrier(0);
+                if (n < 2) scale_w(3, n);
                 if (st + 2 < nsteps) {
 #pragma unroll
                     for (int c = n; c < NV; c += 4 * TB) issue_one(st + 2, d, c);
@@ -379,7 +415,11 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
 #pragma unroll
             for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) tot[rb][tb][v] = __builtin_fmaf(acc[rb][tb][v], sc[tb], tot[rb][tb][v]);
+                for (int v = 0; v < 16; ++v) {
+                    float t = acc[0][rb][tb][v];
+                    if (NP == 2) t = __builtin_fmaf(acc[NP - 1][rb][tb][v], 1.0f / MM_LO, t);
+                    tot[rb][tb][v] = __builtin_fmaf(t, sc[tb], tot[rb][tb][v]);
+                }
     }
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
@@ -463,12 +503,14 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
                 for (int v = 0; v < 16; ++v) acc[tb][v] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const mm_h8 a = mm_frag<BITS>(s.w[q], i, p.xm);
+                mm_h8 a = mm_frag<BITS>(s.w[q], i, p.xm);
 #pragma unroll
-                for (int part = 0; part < 2; ++part)
+                for (int part = 0; part < 2; ++part) {
+                    if (part) a = mm_frag_lo(a);
 #pragma unroll
                     for (int tb = 0; tb < TB; ++tb)
                         acc[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, s.x[tb][i][part], acc[tb], 0, 0, 0);
+                }
             }
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb)
@@ -654,13 +696,10 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
         mm_h8 hi[2], lo[2];
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
+            float v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float v = ldexpf(x[mm_few_x<BITS>(c, i)], -a);
-                hi[c][i] = (_Float16)v;
-                lo[c][i] = (_Float16)__builtin_fmaf((float)hi[c][i], -1.0f, v);
-            }
-            lo[c] = mm_lo(lo[c]);
+            for (int i = 0; i < 8; ++i) v[i] = x[mm_few_x<BITS>(c, i)];
+            mm_split(v, a, hi[c], lo[c]);
         }
         const float sc = ldexpf(1.0f, a);
 #pragma unroll
@@ -672,7 +711,7 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
             for (int i = 0; i < 2; ++i) {
                 const mm_h8 f = mm_few_frag<BITS>(o, i, p.xm);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(f, hi[i], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(f, lo[i], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(mm_frag_lo(f), lo[i], acc, 0, 0, 0);
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v) tot[q][v] = __builtin_fmaf(acc[v], sc, tot[q][v]);

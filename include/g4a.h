@@ -333,10 +333,15 @@ int g4a_linear(g4a_ctx *ctx, const float *w, uint32_t N, uint32_t K, const float
  * 64 run the word-parallel kernel (HBM-bound, f32 sums in another order than the
  * reference's, within f32 reordering error); with M >= 2 (long rows and tall
  * weights: M >= 5), K % 64 == 0 and an 8-byte aligned qbytes they run on the matrix
- * cores instead (x split into two fp16 parts scaled by powers of two, to 2^-24 of
- * its value, from M = 16 in the context's workspace; f32 accumulation, the same
- * error bound; M >= 16 with K <= 256, or where the workspace cannot grow: three bf16
- * parts and exact products). g4a_linear_q with M <= 2 (8 from 64 MiB), one scale
+ * cores instead: x split into two fp16 parts scaled by powers of two, which hold an
+ * activation to 2^-23 of its value (an f32 in four is rounded, in its last bit) if it
+ * is within 2^-27 of the largest of its row's 256 (M <= 16: 64) neighbours, and to
+ * 2^-50 of that largest if it is smaller; f32 accumulation, the same error bound for
+ * activations in that range. From M = 16 the parts live in the context's workspace
+ * (as large as x, 256 MiB at most), so the first such call may allocate and wait for
+ * the stream; M >= 16 with K <= 256, or where the workspace cannot grow (a capture, a
+ * full device), runs on three bf16 parts, which sum to x exactly. g4a_linear_q with
+ * M <= 2 (8 from 64 MiB), one scale
  * per row, rows of a multiple of 128 bytes, K <= 4096 (K % 64 == 0), a 16-byte
  * aligned qbytes and at least 16 MB of packed weights (the lm_head) runs on the
  * int8 matrix cores with x cut into exact digits: within a few f32 ulps of the

@@ -108,6 +108,29 @@ def test_scales_apart_and_non_finite_rows(ctx, M):
     assert np.array_equal(got[5], oracle.linear_q(x[5:6], w)[0], equal_nan=True)
 
 
+@pytest.mark.parametrize("bits,signed", [(4, False), (2, False), (8, True)])
+@pytest.mark.parametrize("M", [9, 20, 400])
+def test_activations_beside_outliers_keep_their_bits(ctx, M, bits, signed):
+    # one |x| of 2^26 times the others in every 64 k, where every weight is 0: the outputs are
+    # sums of the others, held to the bound of f32 sums of those alone
+    N, K = 2048, 1024
+    qb, sc, g = synth.quant_weight(13, N, K, bits, signed_i8=signed, group_size=None)
+    qb = np.array(qb, np.uint8).reshape(N, -1)
+    x = synth.normal_f32(14, 1, M * K).reshape(M, K).copy()
+    per = 8 // bits
+    for k in range(5, K, 64):
+        shift = bits * (k % per)
+        zero = 0 if signed else (1 << (bits - 1)) << shift
+        qb[:, k // per] = (qb[:, k // per] & (0xFF ^ (((1 << bits) - 1) << shift))) | zero
+        x[:, k] = np.float32(2.0 ** 26)
+    w = oracle.QWeight(qb, sc, N, K, bits, signed, g)
+    print(f"[gpu] M={M} b{bits}", flush=True)
+    with Dev(ctx) as d:
+        y = d.empty((M, N))
+        ctx.linear_q(d.w(w), d.arr(x).ptr, y.ptr, M)
+        _check_sum(y.to_host(), oracle.linear_q(x, w), _bound(x, w), f"M={M} b{bits}")
+
+
 @pytest.mark.parametrize("M", [3, 8, 9])
 def test_rows_of_a_large_weight(ctx, M):
     # 64 MiB and more of packed weights: pairs of rows on the int8 matrix cores up to 8 rows
