@@ -130,8 +130,8 @@ struct g4a_ctx {
     hipFunction_t linear_words[3][3][3] = {};  // [bits 2/4/8][(MT, RU) = (1, 2), (1, 8), (4, 4)][mode]
     hipFunction_t linear_elem[3] = {};         // [mode]
     hipFunction_t linear_mfma[3][2][3] = {};   // [bits 2/4/8][64 / 128 weight rows per tile][mode]: M >= 16
-    hipFunction_t linear_mm[5][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead
-    hipFunction_t linear_few[2][3][3] = {};    // [16 / 64 rows a workgroup][bits][mode]: at most 16 activation rows
+    hipFunction_t linear_mm[5][3][3] = {};     // [form][bits 2/4/8][mode]: fp16 parts of x split ahead (linear_mm_built)
+    hipFunction_t linear_few[2][3][3] = {};    // [16 / 32 rows a workgroup][bits][mode]: at most 16 activation rows
     hipFunction_t linear_few16[3] = {};        // [bits]: mode 0, 16 rows a workgroup of 16 waves
     hipFunction_t split_x[3] = {};             // [bits 2/4/8]: the split
     hipFunction_t linear_i8[3][2] = {};        // [bits 2/4/8][M = 1, 2]: int8 matrix cores, mode 0
@@ -259,6 +259,11 @@ int get_fn(g4a_ctx* ctx, hipFunction_t* f, const char* name) {
     if (e != hipSuccess) return fail(ctx, G4A_E_MODULE, "kernel %s missing from code object: %s", name, hipGetErrorString(e));
     return G4A_OK;
 }
+
+// The forms there are (bi: 2 / 4 / 8 bits). At 8 bits form 1 and form 2 of two weights
+// are never the cheapest by MM_FORMS: the former has one workgroup a CU (LDS), the latter
+// spills registers.
+bool linear_mm_built(int form, int bi, int mode) { return bi != 2 || (form != 1 && (form != 2 || mode != 1)); }
 
 // Gives the workspace up: freed, or kept for the live graphs that replay with it.
 // With no graph live, those kept for earlier graphs are freed too.
@@ -791,6 +796,7 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
                     if (int rc = get_fn(ctx, &ctx->linear_few[r][b][m], name)) return bail(rc);
                 }
                 for (int f = 0; f < 5; ++f) {
+                    if (!linear_mm_built(f, b, m)) continue;
                     snprintf(name, sizeof name, "g4a_linear_mm_%d_b%d_mode%d", f, bits[b], m);
                     if (int rc = get_fn(ctx, &ctx->linear_mm[f][b][m], name)) return bail(rc);
                 }
@@ -1746,7 +1752,7 @@ MmForm linear_mm_choose(const g4a_ctx* ctx, int mode, int bi, uint32_t M, uint32
     MmForm best = MM_FORMS[3];
     float least = 3.0e38f;
     for (MmForm f : MM_FORMS) {
-        if (f.tile && !tiles) continue;
+        if ((f.tile && !tiles) || !linear_mm_built(f.form, bi, mode)) continue;
         if (mode == 1 && f.tile) f.rows /= 2;
         const uint64_t wgs = uint64_t((N + f.rows - 1) / f.rows) * ((M + f.toks - 1) / f.toks);
         const uint64_t r = (wgs + cus - 1) / cus;

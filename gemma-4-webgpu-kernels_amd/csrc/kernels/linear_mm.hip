@@ -180,6 +180,15 @@ __device__ __forceinline__ void mm_load_w(const uint8_t* src, uint32_t (&w)[BITS
     }
 }
 
+// A step's offset kept in scalar registers, so that the address is a scalar base plus a
+// lane offset (the compiler would keep a vector address per lane and advance it: eight
+// registers more than the 8-bit blocks have, which then spilled: [1536, 6144] M = 120
+// 27.6 us, 22.6 without).
+__device__ __forceinline__ size_t mm_scalar(size_t offset) {
+    asm("" : "+s"(offset));
+    return offset;
+}
+
 // One output (or four along n): the epilogue of modes 0, 1, 2 as in linear_q.hip.
 template <int MODE>
 __device__ __forceinline__ float mm_out(float v, float v2, float bcol) {
@@ -458,17 +467,23 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
     const uint32_t nblk = (p.M + 31) / 32, tb0 = blockIdx.y * TB;
     const uint32_t nsteps = p.K / 64, nseg = (p.K + MM_SEG - 1) / MM_SEG;
     const uint32_t n0 = blockIdx.x * 32 * RB;
+    // scalar bases, which the step moves, and lane offsets (as linear_mm_tile)
     const uint8_t* wp[NR];
+    uint32_t woff[RB];
 #pragma unroll
-    for (int q = 0; q < NR; ++q)
-        wp[q] = (q >= RB ? p.wb2 : p.wb) + (size_t)min(n0 + 32 * (q % RB) + rl, p.N - 1) * p.row_bytes + h * 4 * BITS;
-    const mm_h8* xp[TB];
-    const float* scp[TB];
+    for (int q = 0; q < NR; ++q) {
+        const uint32_t row = min(n0 + 32 * (q % RB), p.N - 1);
+        wp[q] = (q >= RB ? p.wb2 : p.wb) + (size_t)row * p.row_bytes;
+        woff[q % RB] = min((uint32_t)rl, p.N - 1 - row) * p.row_bytes + h * 4 * BITS;
+    }
+    const uint8_t* xp[TB];
+    const uint8_t* scp[TB];
+    const uint32_t xoff = 16 * (256 * h + rl), soff = 4 * rl;
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
         const uint32_t b = min(tb0 + tb, nblk - 1);
-        xp[tb] = reinterpret_cast<const mm_h8*>(p.xs) + (size_t)b * p.K * 8 + 256 * h + rl;
-        scp[tb] = p.xscale + (size_t)b * nseg * 32 + rl;
+        xp[tb] = reinterpret_cast<const uint8_t*>(p.xs) + (size_t)b * p.K * 128;
+        scp[tb] = reinterpret_cast<const uint8_t*>(p.xscale + (size_t)b * nseg * 32);
     }
     struct Step {
         uint32_t w[NR][BITS];
@@ -478,14 +493,16 @@ __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
     auto load = [&](Step& s, uint32_t st) {
         if (st >= nsteps) return;  // (the step index is the wave's: no divergence)
 #pragma unroll
-        for (int q = 0; q < NR; ++q) mm_load_w<BITS>(wp[q] + (size_t)st * 8 * BITS, s.w[q]);
+        for (int q = 0; q < NR; ++q) mm_load_w<BITS>(wp[q] + mm_scalar((size_t)st * 8 * BITS) + woff[q % RB], s.w[q]);
 #pragma unroll
         for (int tb = 0; tb < TB; ++tb) {
+            const uint8_t* const xs = xp[tb] + mm_scalar((size_t)st * 8192);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int part = 0; part < 2; ++part) s.x[tb][i][part] = xp[tb][(size_t)st * 512 + (2 * i + part) * 32];
-            s.sc[tb] = scp[tb][(st >> 2) * 32];
+                for (int part = 0; part < 2; ++part)
+                    s.x[tb][i][part] = *reinterpret_cast<const mm_h8*>(xs + xoff + (2 * i + part) * 512);
+            s.sc[tb] = *reinterpret_cast<const float*>(scp[tb] + mm_scalar((size_t)(st >> 2) * 128) + soff);
         }
     };
     float tot[NB][16];
@@ -753,20 +770,24 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
 
 // Forms 0, 1, 4: tiles of 128 tokens x 256 / 128 rows and 64 tokens x 128 rows; 2, 3:
 // k-split blocks of 32 tokens x 64 / 32 rows (in mode 1 the tiles share their rows
-// between the weights, the blocks hold as many of each).
+// between the weights, the blocks hold as many of each). At 8 bits form 1, whose two
+// workgroups a CU the weights' LDS rules out, and form 2 of two weights, which spills,
+// are not built (linear_mm_choose).
 #define G4A_MM(B, MODE)                                                                                           \
-    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_0_b##B##_mode##MODE(G4aLinearMmParams p) {      \
-        linear_mm_tile<B, MODE, 8, 2>(p);                                                                            \
+    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_0_b##B##_mode##MODE(G4aLinearMmParams p) {    \
+        linear_mm_tile<B, MODE, 8, 2>(p);                                                                         \
     }                                                                                                             \
-    extern "C" __global__ __launch_bounds__(256, 2) void g4a_linear_mm_1_b##B##_mode##MODE(G4aLinearMmParams p) {      \
-        linear_mm_tile<B, MODE, 4, 2>(p);                                                                            \
-    }                                                                                                             \
-    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_2_b##B##_mode##MODE(G4aLinearMmParams p) {      \
-        linear_mm_ksplit<B, MODE, 2, 1>(p);                                                       \
-    }                                                                                                             \
-    extern "C" __global__ __launch_bounds__(512, MODE == 1 ? 2 : 4) void g4a_linear_mm_3_b##B##_mode##MODE(         \
+    extern "C" __global__ __launch_bounds__(512, MODE == 1 ? 2 : 4) void g4a_linear_mm_3_b##B##_mode##MODE(       \
         G4aLinearMmParams p) {                                                                                    \
         linear_mm_ksplit<B, MODE, 1, 1>(p);                                                                       \
+    }
+#define G4A_MM_1(B, MODE)                                                                                         \
+    extern "C" __global__ __launch_bounds__(256, 2) void g4a_linear_mm_1_b##B##_mode##MODE(G4aLinearMmParams p) { \
+        linear_mm_tile<B, MODE, 4, 2>(p);                                                                         \
+    }
+#define G4A_MM_2(B, MODE)                                                                                         \
+    extern "C" __global__ __launch_bounds__(512) void g4a_linear_mm_2_b##B##_mode##MODE(G4aLinearMmParams p) {    \
+        linear_mm_ksplit<B, MODE, 2, 1>(p);                                                                       \
     }
 #define G4A_MM_T64(B, MODE)                                                                                       \
     extern "C" __global__ __launch_bounds__(256, 3) void g4a_linear_mm_4_b##B##_mode##MODE(G4aLinearMmParams p) {   \
@@ -789,3 +810,6 @@ __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
 G4A_MM_SET(2)
 G4A_MM_SET(4)
 G4A_MM_SET(8)
+G4A_MM_1(2, 0) G4A_MM_1(2, 1) G4A_MM_1(2, 2) G4A_MM_1(4, 0) G4A_MM_1(4, 1) G4A_MM_1(4, 2)
+G4A_MM_2(2, 0) G4A_MM_2(2, 1) G4A_MM_2(2, 2) G4A_MM_2(4, 0) G4A_MM_2(4, 1) G4A_MM_2(4, 2)
+G4A_MM_2(8, 0) G4A_MM_2(8, 2)
