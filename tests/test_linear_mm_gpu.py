@@ -1,12 +1,13 @@
-"""Projections of 2 and more rows on split activations (linear_mm_*): every form
-(128-token tiles of 256 and 128 rows, 64-token ones of 128, 32-token k-split blocks of 64 and 32 rows,
-16-token blocks of 32 and 16), the int8 kernel over pairs of rows of a large weight,
-at ragged edges of its tiles and steps, every weight format and epilogue, against
-the CPU oracle within the bound of another f32 summation order
-(2e-6 * sum |x w| + 1e-7 per output, as tests/test_linear_gpu.py derives it);
-activations far apart in scale within a row, whose segments scale apart; rows
-holding an inf or NaN; and a capture on a context whose workspace is too small
-for the split, which runs the kernel that needs none."""
+"""Projections of 2 and more rows on split activations (linear_mm_*): every kernel
+of them (128-token tiles of 256 and 128 rows, 64-token ones of 128, 32-token k-split
+blocks of 64 and 32 rows, 16-token blocks of 32 and 16; every weight format and
+epilogue) at ragged edges of its tiles and steps (EVERY_KERNEL, whose routes
+tests/test_linear_routes_host.py asserts without a GPU), the int8 kernel over pairs
+of rows of a large weight, against the CPU oracle within the bound of another f32
+summation order (2e-6 * sum |x w| + 1e-7 per output, as tests/test_linear_gpu.py
+derives it); activations far apart in scale within a row, whose segments scale apart,
+and beside outliers; rows holding an inf or NaN; and a capture on a context whose
+workspace is too small for the split, which runs the kernel that needs none."""
 import numpy as np
 import pytest
 
@@ -64,6 +65,109 @@ def test_forms_match_the_oracle(ctx, op, N, K, M, bits, signed):
             b = synth.normal_f32(4, 2, M * (N + 5)).reshape(M, N + 5)
             ctx.linear_q_gelu_mul_cols(dw, dx.ptr, d.arr(b).ptr, N + 5, 3, y.ptr, M)
             _check_fused(y.to_host(), x, w, None, b, 3, name)
+
+
+# kernel, entry point, N, K, M, bits: no multiple of a tile or of a scale's segment
+EVERY_KERNEL = [
+    ("0_b2_mode0", "linear", 2946, 1728, 1392, 2),
+    ("0_b2_mode1", "geglu", 1635, 320, 1933, 2),
+    ("0_b2_mode2", "gelu_cols", 2575, 320, 2382, 2),
+    ("0_b4_mode0", "linear", 1537, 1600, 2644, 4),
+    ("0_b4_mode1", "geglu", 1594, 320, 2087, 4),
+    ("0_b4_mode2", "gelu_cols", 3545, 320, 1752, 4),
+    ("0_b8_mode0", "linear", 2598, 832, 1752, 8),
+    ("0_b8_mode1", "geglu", 1261, 832, 1610, 8),
+    ("0_b8_mode2", "gelu_cols", 3207, 1088, 1228, 8),
+    ("1_b2_mode0", "linear", 2931, 1152, 2727, 2),
+    ("1_b2_mode1", "geglu", 2461, 896, 1544, 2),
+    ("1_b2_mode2", "gelu_cols", 1915, 640, 4207, 2),
+    ("1_b4_mode0", "linear", 1822, 640, 4178, 4),
+    ("1_b4_mode1", "geglu", 1251, 640, 4347, 4),
+    ("1_b4_mode2", "gelu_cols", 3103, 704, 3542, 4),
+    ("2_b2_mode0", "linear", 409, 896, 610, 2),
+    ("2_b2_mode1", "geglu", 519, 320, 1456, 2),
+    ("2_b2_mode2", "gelu_cols", 407, 960, 621, 2),
+    ("2_b4_mode0", "linear", 398, 832, 662, 4),
+    ("2_b4_mode1", "geglu", 555, 320, 1384, 4),
+    ("2_b4_mode2", "gelu_cols", 511, 896, 613, 4),
+    ("2_b8_mode0", "linear", 547, 640, 1377, 8),
+    ("2_b8_mode2", "gelu_cols", 939, 640, 903, 8),
+    ("3_b2_mode0", "linear", 27, 384, 17, 2),
+    ("3_b2_mode1", "geglu", 22, 320, 24, 2),
+    ("3_b2_mode2", "gelu_cols", 27, 320, 17, 2),
+    ("3_b4_mode0", "linear", 25, 320, 17, 4),
+    ("3_b4_mode1", "geglu", 23, 320, 18, 4),
+    ("3_b4_mode2", "gelu_cols", 22, 448, 17, 4),
+    ("3_b8_mode0", "linear", 26, 320, 18, 8),
+    ("3_b8_mode1", "geglu", 25, 320, 21, 8),
+    ("3_b8_mode2", "gelu_cols", 23, 320, 18, 8),
+    ("4_b2_mode0", "linear", 839, 320, 1862, 2),
+    ("4_b2_mode1", "geglu", 525, 320, 2089, 2),
+    ("4_b2_mode2", "gelu_cols", 2386, 320, 645, 2),
+    ("4_b4_mode0", "linear", 1237, 320, 1328, 4),
+    ("4_b4_mode1", "geglu", 551, 320, 1963, 4),
+    ("4_b4_mode2", "gelu_cols", 1413, 448, 1076, 4),
+    ("4_b8_mode0", "linear", 1011, 320, 1079, 8),
+    ("4_b8_mode1", "geglu", 389, 320, 2014, 8),
+    ("4_b8_mode2", "gelu_cols", 2246, 320, 466, 8),
+    ("few_r1_b2_mode0", "linear", 21, 64, 2, 2),
+    ("few_r1_b2_mode1", "geglu", 8585, 64, 2, 2),
+    ("few_r1_b2_mode2", "gelu_cols", 22, 64, 4, 2),
+    ("few_r1_b4_mode0", "linear", 21, 64, 3, 4),
+    ("few_r1_b4_mode1", "geglu", 8302, 64, 2, 4),
+    ("few_r1_b4_mode2", "gelu_cols", 25, 64, 2, 4),
+    ("few_r1_b8_mode0", "linear", 22, 64, 2, 8),
+    ("few_r1_b8_mode1", "geglu", 8810, 64, 3, 8),
+    ("few_r1_b8_mode2", "gelu_cols", 21, 64, 2, 8),
+    ("few_r2_b2_mode0", "linear", 16861, 64, 5, 2),
+    ("few_r2_b2_mode1", "geglu", 23, 64, 4, 2),
+    ("few_r2_b2_mode2", "gelu_cols", 17467, 64, 5, 2),
+    ("few_r2_b4_mode0", "linear", 16514, 64, 7, 4),
+    ("few_r2_b4_mode1", "geglu", 21, 64, 2, 4),
+    ("few_r2_b4_mode2", "gelu_cols", 16431, 64, 6, 4),
+    ("few_r2_b8_mode0", "linear", 17027, 64, 5, 8),
+    ("few_r2_b8_mode1", "geglu", 21, 64, 3, 8),
+    ("few_r2_b8_mode2", "gelu_cols", 19687, 64, 5, 8),
+    ("few_w16_b2_mode0", "linear", 21, 1088, 3, 2),
+    ("few_w16_b4_mode0", "linear", 21, 1152, 2, 4),
+    ("few_w16_b8_mode0", "linear", 21, 1088, 2, 8),
+]
+
+
+def _ends(n, count, seed):
+    """Indices at both ends of n and some between."""
+    if n <= 3 * count:
+        return np.arange(n)
+    mid = np.random.default_rng(seed).choice(np.arange(count, n - count), count, replace=False)
+    return np.sort(np.r_[0:count, n - count:n, mid])
+
+
+@pytest.mark.parametrize("kernel,op,N,K,M,bits", EVERY_KERNEL)
+def test_every_kernel_matches_the_oracle(ctx, kernel, op, N, K, M, bits):
+    print(f"[gpu] {kernel} {op} N={N} K={K} M={M}", flush=True)
+    signed = bits == 8 and N % 2 == 1  # 8-bit rows of both kinds
+    rows, toks = _ends(N, 150, 1), _ends(M, 70, 2)
+    w, x = _qw(1, N, K, bits, signed, None), synth.normal_f32(2, 1, M * K).reshape(M, K)
+    xt = np.ascontiguousarray(x[toks])
+
+    def part(w):
+        qb = np.ascontiguousarray(np.asarray(w.qbytes, np.uint8).reshape(N, -1)[rows])
+        return oracle.QWeight(qb, w.scales.reshape(N, -1)[rows], rows.size, K, bits, signed, K)
+
+    with Dev(ctx) as d:
+        dw, dx, y = d.w(w), d.arr(x), d.empty((M, N))
+        if op == "linear":
+            ctx.linear_q(dw, dx.ptr, y.ptr, M)
+            _check_sum(y.to_host()[np.ix_(toks, rows)], oracle.linear_q(xt, part(w)), _bound(xt, part(w)), kernel)
+        elif op == "geglu":
+            w2 = _qw(3, N, K, bits, signed, None)
+            ctx.linear_q_geglu(dw, d.w(w2), dx.ptr, y.ptr, M)
+            _check_fused(y.to_host()[np.ix_(toks, rows)], xt, part(w), part(w2), None, 0, kernel)
+        else:
+            b = synth.normal_f32(4, 2, M * (N + 5)).reshape(M, N + 5)
+            ctx.linear_q_gelu_mul_cols(dw, dx.ptr, d.arr(b).ptr, N + 5, 3, y.ptr, M)
+            _check_fused(y.to_host()[np.ix_(toks, rows)], xt, part(w), None, np.ascontiguousarray(b[np.ix_(toks, rows + 3)]),
+                         0, kernel)
 
 
 @pytest.mark.parametrize("bits,signed", [(4, False), (8, True), (2, False)])
