@@ -39,7 +39,7 @@ constexpr float PREFILL_TAU_LOGN = 2.0f;
 // The prefill split's cost model (prefill_split), in the time of one 16-key tile
 // of a workgroup (1.3 us at head_dim 256, 2.6 at 512): a workgroup's fixed cost,
 // the merge launch, a partial slot's write and read; the fewest tiles worth a
-// share; and the most partial slots of a call (132 KiB each at head_dim 512).
+// share; and the most partial slots of a call (129 KiB each at head_dim 512).
 constexpr float PREFILL_WG_TILES_256 = 18.0f;
 constexpr float PREFILL_WG_TILES_512 = 11.0f;
 constexpr float PREFILL_MERGE_TILES = 3.0f;
@@ -349,26 +349,51 @@ struct PrefillSplit {
 };
 
 // A query block's workgroups when its heaviest block has `most`: shares of at
-// most `tpi` tiles, in steps that keep the counts to G4A_PF_CLASSES.
-uint32_t prefill_shares(uint32_t nt, uint32_t tpi, uint32_t most) {
-    const uint32_t step = (most + G4A_PF_CLASSES - 2) / (G4A_PF_CLASSES - 1);
-    const uint32_t n = (nt + tpi - 1) / tpi;
-    return n <= 1 ? 1 : std::min(most, (n + step - 1) / step * step);
-}
+// most `tpi` tiles, in steps that keep the counts to G4A_PF_CLASSES. (Quotients by
+// reciprocals: a whole number plus a half is far from the next one.)
+struct PrefillShares {
+    uint32_t tpi, most, step;
+    double per_tpi, per_step;
+    PrefillShares(uint32_t tpi_, uint32_t most_)
+        : tpi(tpi_), most(most_), step((most_ + G4A_PF_CLASSES - 2) / (G4A_PF_CLASSES - 1)), per_tpi(1.0 / tpi_),
+          per_step(1.0 / step) {}
+    uint32_t operator()(uint32_t nt) const {
+        const uint32_t n = uint32_t((double(nt) + (tpi - 0.5)) * per_tpi);
+        return n <= 1 ? 1 : std::min(most, uint32_t((n + (step - 0.5)) * per_step) * step);
+    }
+};
 
-// Splits every block at `tpi` tiles a share, `most` shares at most.
-PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, uint32_t tpi, uint32_t most) {
+// Splits every block by `shares`.
+PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, const PrefillShares& shares) {
     PrefillSplit sp;
     // from the first block on, the share count never decreases (a window's tile
     // counts move up and down by one with its alignment)
     uint32_t nb[G4A_PF_CLASSES] = {}, ns[G4A_PF_CLASSES] = {1}, n = 0;
-    for (uint32_t b = 0; b < NB; ++b) {
-        const uint32_t s = prefill_shares(tiles(b), tpi, most);
-        if (s > ns[n]) {
-            if (nb[n]) ++n;
-            ns[n] = s;
+    if (shares.most == 1) {
+        nb[0] = NB;
+    } else if (tiles.a->sliding_window == 0) {
+        // without a window later blocks never have fewer tiles: each class's end by bisection
+        for (uint32_t b = 0; b < NB; ++n) {
+            ns[n] = shares(tiles(b));
+            uint32_t lo = b + 1, hi = NB;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (shares(tiles(mid)) > ns[n]) hi = mid;
+                else lo = mid + 1;
+            }
+            nb[n] = lo - b;
+            b = lo;
         }
-        ++nb[n];
+        --n;
+    } else {
+        for (uint32_t b = 0; b < NB; ++b) {
+            const uint32_t s = shares(tiles(b));
+            if (s > ns[n]) {
+                if (nb[n]) ++n;
+                ns[n] = s;
+            }
+            ++nb[n];
+        }
     }
     for (int c = int(n); c >= 0; --c) {
         sp.nb[sp.ncls] = nb[c];
@@ -386,67 +411,104 @@ PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, uint32_t t
 // at a scale of PF_SIM_CUS; a split block adds the traffic of its partials and a
 // merge launch. Tried: share counts of the heaviest block spaced by about a
 // quarter, the one that just fills the CUs, and halving the blocks above the
-// mean, on up to 64 sampled blocks.
+// mean, on up to 64 sampled blocks. A count whose largest share, or whose work
+// divided over the CUs, already takes longer than the best so far is dropped
+// unplayed: the choice takes 0.5 .. 8 us of host time, behind the pre-pass's launch
+// (8 .. 18 us from T = 173 on with every count played, ahead of it, which showed in
+// a lone call).
 // Against a sweep of fixed counts the choice is within 5 % of the best over T =
 // 16 .. 2048 and up to 16000 earlier keys (us, one workgroup a block -> chosen):
 // hd512 T = 173 after 6001 keys 1048 -> 168, 16 after 16000 2639 -> 128, T = 2048
 // 385 -> 317 (363 with the later blocks halved), 231 74 -> 44; hd256 window 512,
 // T = 2048 unchanged, 512 79 -> 46, 120 after 3000 83 -> 43.
-constexpr int PF_SIM_CUS = 32;
+constexpr uint32_t PF_SIM_CUS = 32;
+
+// The played-through launch of `items` workgroups per sampled block, from the last
+// (heaviest) on, in tiles: the time the last CU is done, or any time past `limit`
+// once one passes it. `busy` is a heap, the CU that frees first on top.
+template <typename Shares>
+float prefill_rounds(const uint32_t* nt, uint32_t n, const Shares& shares, float fixed, float each, float limit) {
+    float busy[2 * PF_SIM_CUS + 1];
+    std::fill(busy, busy + PF_SIM_CUS, 0.0f);
+    std::fill(busy + PF_SIM_CUS, busy + 2 * PF_SIM_CUS + 1, 3.0e38f);
+    float due = 0.0f, last = 0.0f;
+    for (uint32_t i = n; i-- > 0;) {
+        const uint32_t s = shares(nt[i]);
+        const float cost = float(nt[i]) / float(s) + fixed;
+        for (due += float(s) * each; due >= 1.0f; due -= 1.0f) {
+            const float t = busy[0] + cost;
+            last = std::max(last, t);
+            if (last > limit) return last;
+            uint32_t at = 0;
+            for (;;) {
+                const uint32_t c = 2 * at + 1 + (busy[2 * at + 2] < busy[2 * at + 1]);
+                if (c >= PF_SIM_CUS || busy[c] >= t) break;
+                busy[at] = busy[c];
+                at = c;
+            }
+            busy[at] = t;
+        }
+    }
+    return last;
+}
 
 PrefillSplit prefill_split(const PrefillTiles& tiles, uint32_t NB, uint32_t Hkv, uint64_t cus, bool d512,
                            uint32_t max_slots) {
     const float fixed = d512 ? PREFILL_WG_TILES_512 : PREFILL_WG_TILES_256;
     const uint32_t n = std::min<uint32_t>(NB, 64);
     uint32_t nt[64], top = std::max(tiles(NB - 1), 1u);
+    uint64_t sum = 0;
     for (uint32_t i = 0; i < n; ++i) {
         nt[i] = tiles(uint32_t((uint64_t(i) * 2 + 1) * NB / (2 * n)));
         top = std::max(top, nt[i]);
+        sum += nt[i];
     }
     const double each = double(NB) * Hkv / n;  // blocks a sample stands for
-    auto rounds = [&](uint32_t tpi, uint32_t most) {
-        float busy[PF_SIM_CUS] = {};
-        const float w = float(each * PF_SIM_CUS / double(cus));
-        float due = 0.0f;
-        for (uint32_t i = n; i-- > 0;) {
-            const uint32_t s = prefill_shares(nt[i], tpi, most);
-            const float cost = float(nt[i]) / float(s) + fixed;
-            for (due += float(s) * w; due >= 1.0f; due -= 1.0f) *std::min_element(busy, busy + PF_SIM_CUS) += cost;
-        }
-        return *std::max_element(busy, busy + PF_SIM_CUS);
-    };
+    const float w = float(each * PF_SIM_CUS / double(cus));
     float best = 3.0e38f;
     uint32_t best_tpi = top, best_most = 1;
+    // the work of `items` workgroups of all sampled blocks over the CUs, less the one not
+    // yet due: no launch of more workgroups than CUs takes less
+    auto spread = [&](double items, float longest) {
+        return 0.999 * ((double(sum) + items * fixed) * w - longest) / PF_SIM_CUS;
+    };
     auto consider = [&](uint32_t tpi, uint32_t most) {
         if (most > 1 && tpi < PREFILL_MIN_SHARE) return;
-        double items = 0, slots = 0;
+        float est = std::max(float(tpi), float(top) / float(most)) + fixed;
+        if (est >= best) return;
+        const double least = uint64_t(tpi) * most >= top ? std::max(double(n), double(sum) / tpi) : double(n);
+        if (least * each > double(cus) && spread(least, est) >= best) return;
+        const PrefillShares shares(tpi, most);
+        uint32_t in_all = 0, in_split = 0;
         for (uint32_t i = 0; i < n; ++i) {
-            const uint32_t s = prefill_shares(nt[i], tpi, most);
-            items += s;
-            if (s > 1) slots += s;
+            const uint32_t s = shares(nt[i]);
+            in_all += s;
+            in_split += s > 1 ? s : 0;
         }
-        items *= each, slots *= each;
+        const double items = in_all * each, slots = in_split * each;
         // (many rounds more than the unsplit launch's gain nothing)
         if (slots > max_slots || (most > 1 && items > 4.0 * double(cus) && items > 1.5 * each * n)) return;
-        float est = std::max(float(tpi), float(top) / float(most)) + fixed;
-        if (items > double(cus)) est = std::max(est, rounds(tpi, most));
-        if (slots > 0) est += PREFILL_MERGE_TILES + float(slots) * PREFILL_SLOT_TILES;
+        const float merge = slots > 0 ? PREFILL_MERGE_TILES + float(slots) * PREFILL_SLOT_TILES : 0.0f;
+        if (est + merge >= best) return;
+        if (items > double(cus)) {
+            if (best < 3.0e38f && spread(in_all, est) + merge >= best) return;
+            est = std::max(est, prefill_rounds(nt, n, shares, fixed, w, best));
+        }
+        est += merge;
         if (est < best) best = est, best_tpi = tpi, best_most = most;
     };
     auto even = [&](uint32_t most) { consider((top + most - 1) / most, most); };
     for (uint32_t most = 1; most <= G4A_PF_MAX_SHARES; most = most < 4 ? most + 1 : most + most / 4) even(most);
     const uint64_t fill = cus / (uint64_t(NB) * Hkv);
     if (fill > 1) even(uint32_t(std::min<uint64_t>(fill, G4A_PF_MAX_SHARES)));
-    uint64_t sum = 0;
-    for (uint32_t i = 0; i < n; ++i) sum += nt[i];
     consider(uint32_t(sum / n) + 1, 2);  // only the blocks above the mean, halved
-    const PrefillSplit sp = prefill_split_at(tiles, NB, best_tpi, best_most);
+    const PrefillSplit sp = prefill_split_at(tiles, NB, PrefillShares(best_tpi, best_most));
     // (the sampled tile counts can miss the limit)
-    return uint64_t(sp.slots) * Hkv <= max_slots ? sp : prefill_split_at(tiles, NB, top, 1);
+    return uint64_t(sp.slots) * Hkv <= max_slots ? sp : prefill_split_at(tiles, NB, PrefillShares(top, 1));
 }
 
 // Bytes of partials g4a_attention_noalloc counts against its static array, which
-// sets what it refuses: at head_dim 512, two 132 KiB halves for each trailing
+// sets what it refuses: at head_dim 512, two 129 KiB halves for each trailing
 // block of more tiles than the average.
 size_t noalloc_partial_bytes(const PrefillTiles& tiles, bool d512) {
     if (!d512) return 0;
@@ -1061,48 +1123,60 @@ int attention_run(g4a_ctx* ctx, const g4a_attn_args* a, const Analysis& an, bool
                                       uint32_t(std::min<size_t>(bytes / slot_bytes, PREFILL_MAX_SLOTS)));
                 return part_off + split.slots * a->Hkv * slot_bytes;
             };
-            size_t need = choose(room);
+            // the pre-pass, which the chosen split does not touch: its launch goes ahead of the
+            // choice wherever its place in the workspace is known by then
+            auto split_kv = [&](void* at) {
+                char* const ws = static_cast<char*>(at);
+                G4aSplitParams sp{};
+                sp.k = a->k;
+                sp.v = a->v;
+                sp.kout = reinterpret_cast<float*>(ws + 256);
+                sp.vout = reinterpret_cast<float*>(ws + 256 + half);
+                sp.kscale = reinterpret_cast<float*>(ws + 256 + 2 * half);
+                sp.vflag = reinterpret_cast<uint32_t*>(ws);
+                sp.k0 = k0;
+                sp.nkeys = nkeys;
+                sp.S = a->S;
+                sp.Hkv = a->Hkv;
+                sp.Dh = a->Dh;
+                sp.ring_cap = a->kv_ring_cap;
+                sp.epoch = next_split_epoch();
+                sp.vis_lo = pl.k_start;
+                sp.vis_hi = pl.k_end;
+                pp.ksplit = sp.kout;
+                pp.kscale = sp.kscale;
+                pp.vsplit = sp.vout;
+                pp.vflag = sp.vflag;
+                pp.split0 = k0;
+                pp.split_n = nkeys;
+                pp.epoch = sp.epoch;
+                pp.part = reinterpret_cast<float*>(ws + part_off);
+                // one block per (16-key tile, kv head) for K, then one thread per 4 dims of a V key quad
+                const uint64_t vthreads = uint64_t(nkeys / 4) * a->Hkv * (a->Dh / 64) * 16;
+                const uint64_t blocks = uint64_t(nkeys / 16) * a->Hkv + (vthreads + 255) / 256;
+                return launch(ctx, ctx->split_kv, dim3(uint32_t(blocks), 1, 1), dim3(256, 1, 1), sp, "split K/V");
+            };
+            void *ws = nullptr, *at = nullptr;
             if (noalloc) {
-                need = part_off + noalloc_partial_bytes(tiles, d512);
-            } else if (const int rc = grow_workspace(ctx, need, false)) {
-                if (rc != G4A_E_NOMEM) return rc;
-                // a capture, which cannot grow the workspace, or a device without the memory:
-                // no more shares than the workspace has room for
-                need = choose(std::max(ctx->workspace_bytes, part_off) - part_off);
+                if (int rc = call_workspace(ctx, part_off + noalloc_partial_bytes(tiles, d512), true, &ws)) return rc;
+                if (int rc = split_kv(ws)) return rc;
+                choose(room);
+            } else {
+                if (part_off <= ctx->workspace_bytes) {
+                    at = ctx->workspace;
+                    if (int rc = split_kv(at)) return rc;
+                }
+                size_t need = choose(room);
+                if (const int rc = grow_workspace(ctx, need, false)) {
+                    if (rc != G4A_E_NOMEM) return rc;
+                    // a capture, which cannot grow the workspace, or a device without the memory:
+                    // no more shares than the workspace has room for
+                    need = choose(std::max(ctx->workspace_bytes, part_off) - part_off);
+                }
+                if (int rc = call_workspace(ctx, need, false, &ws)) return rc;
+                if (ws != at)  // the workspace was too small, or grew for the partials
+                    if (int rc = split_kv(ws)) return rc;
             }
-            void* wsp = nullptr;
-            if (int rc = call_workspace(ctx, need, noalloc, &wsp)) return rc;
-            char* const ws = static_cast<char*>(wsp);
-            G4aSplitParams sp{};
-            sp.k = a->k;
-            sp.v = a->v;
-            sp.kout = reinterpret_cast<float*>(ws + 256);
-            sp.vout = reinterpret_cast<float*>(ws + 256 + half);
-            sp.kscale = reinterpret_cast<float*>(ws + 256 + 2 * half);
-            sp.vflag = reinterpret_cast<uint32_t*>(ws);
-            sp.k0 = k0;
-            sp.nkeys = nkeys;
-            sp.S = a->S;
-            sp.Hkv = a->Hkv;
-            sp.Dh = a->Dh;
-            sp.ring_cap = a->kv_ring_cap;
-            sp.epoch = next_split_epoch();
-            sp.vis_lo = pl.k_start;
-            sp.vis_hi = pl.k_end;
-            // one block per (16-key tile, kv head) for K, then one thread per 4 dims of a V key quad
-            const uint64_t vthreads = uint64_t(nkeys / 4) * a->Hkv * (a->Dh / 64) * 16;
-            const uint64_t blocks = uint64_t(nkeys / 16) * a->Hkv + (vthreads + 255) / 256;
-            if (int rc = launch(ctx, ctx->split_kv, dim3(uint32_t(blocks), 1, 1), dim3(256, 1, 1), sp,
-                                "split K/V"))
-                return rc;
-            pp.ksplit = sp.kout;
-            pp.kscale = sp.kscale;
-            pp.vsplit = sp.vout;
-            pp.vflag = sp.vflag;
-            pp.split0 = k0;
-            pp.split_n = nkeys;
-            pp.epoch = sp.epoch;
-            pp.part = reinterpret_cast<float*>(ws + part_off);
         }
         pp.part_slots = split.slots;
         pp.ncls = split.ncls;
