@@ -416,11 +416,13 @@ PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, const Pref
 // unplayed: the choice takes 0.5 .. 8 us of host time, behind the pre-pass's launch
 // (8 .. 18 us from T = 173 on with every count played, ahead of it, which showed in
 // a lone call).
-// Against a sweep of fixed counts the choice is within 5 % of the best over T =
-// 16 .. 2048 and up to 16000 earlier keys (us, one workgroup a block -> chosen):
-// hd512 T = 173 after 6001 keys 1048 -> 168, 16 after 16000 2639 -> 128, T = 2048
-// 385 -> 317 (363 with the later blocks halved), 231 74 -> 44; hd256 window 512,
-// T = 2048 unchanged, 512 79 -> 46, 120 after 3000 83 -> 43.
+// Against a sweep of fixed counts (72 calls of T = 16 .. 2048 and up to 16000 earlier
+// keys, both head_dims, with and without a window) the choice is within 5 % of the best,
+// 6 % at 300 tokens and 9 % (3 us) at 64 of head_dim 512 (us, one workgroup a block ->
+// chosen): hd512 T = 173 after 6001 keys 1029 -> 159, 16 after 16000 2639 -> 123, T = 2048
+// 357 -> 297, 231 74 -> 44; hd256 window 512, T = 2048 unchanged, 512 79 -> 45, 120 after
+// 3000 83 -> 41. A few workgroups more than CUs cost a second round, which a part of one
+// left over in the play must count for: 513 after 3000 312 -> 240, 700 89 -> 72.
 constexpr uint32_t PF_SIM_CUS = 32;
 
 // The played-through launch of `items` workgroups per sampled block, from the last
@@ -435,7 +437,9 @@ float prefill_rounds(const uint32_t* nt, uint32_t n, const Shares& shares, float
     for (uint32_t i = n; i-- > 0;) {
         const uint32_t s = shares(nt[i]);
         const float cost = float(nt[i]) / float(s) + fixed;
-        for (due += float(s) * each; due >= 1.0f; due -= 1.0f) {
+        due += float(s) * each;
+        if (i == 0) due = std::ceil(due - 0.01f);  // a part of a workgroup left over is one more
+        for (; due >= 1.0f; due -= 1.0f) {
             const float t = busy[0] + cost;
             last = std::max(last, t);
             if (last > limit) return last;

@@ -41,6 +41,17 @@ def test_shares(ctx, T, past, Dh, window, workgroups, merge):
     assert got[1].gx == workgroups and (not merge or got[2].gx == merge)
 
 
+def test_no_second_round_for_a_few_workgroups(ctx):
+    # 513 .. 700 tokens in shares of 257 .. 263 workgroups on 256 CUs took up to a half more than
+    # in fewer shares; a head_dim, a window and earlier keys of each kind
+    for Dh, window in ((256, 0), (256, 512), (512, 0)):
+        for past in (0, 100, 1000, 3000, 6001):
+            for T in range(17, 800, 29):
+                ctx.attention_batch(ctx.prepare_batch([_args(T, past, Dh, window)]))
+                grid = next(x.gx for x in hip.launches() if "prefill2" in x.name)
+                assert not 256 < grid < 280, (T, past, Dh, window, grid)
+
+
 def test_a_workspace_that_grows_for_the_partials_has_the_splits_too():
     with hip.binding().Context(0) as c:
         c.linear_q(hip.weight(64, 2048, 4), PTR, PTR, 3700)  # 30 MB of workspace: the K/V splits' place, 16.8 MB
