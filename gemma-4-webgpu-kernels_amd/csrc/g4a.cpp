@@ -1804,10 +1804,12 @@ LinearChoice choose_linear(const g4a_ctx* ctx, int mode, const g4a_qweight* w, c
 
 // The linear_mm form of a call: the one whose workgroups take the least time. A
 // form's r = ceil(workgroups / CUs) workgroups per CU take r * (step us per 64 k +
-// fixed us), or for r = 1, with the CU to itself, solo (measured with every CU busy,
-// 4-bit; 8-bit weights take `wide` times as long). Against every form at M = 64 ..
-// 2048 of [2048, 1536], [1536, 6144], [1536, 12288] and gate + up [6144, 1536],
-// [12288, 1536] weights at 2, 4 and 8 bits, the choice is within 10 % of the best.
+// fixed us), or for r = 1, with the CU to itself, solo (fitted to calls with every CU
+// busy; 8-bit weights take `wide` times as long). Against every form at 13 M = 17 ..
+// 2048 of [2048, 1536], [1536, 2048 .. 12288], [4096, 1536], [256, 1536] and gate + up
+// [6144, 1536], [12288, 1536] weights at 2, 4 and 8 bits (390 calls), the choice is within
+// 5 % of the best in 375 and within 10 % in all but 256 weight rows at 800 .. 1024 tokens
+// (2 us of 14).
 struct MmForm {
     int form;
     uint32_t rows, toks, threads;  // weight rows (of each weight) and tokens of a workgroup
@@ -1818,11 +1820,11 @@ struct MmForm {
     float wide;
 };
 constexpr MmForm MM_FORMS[5] = {
-    {0, 256, 128, 512, true, {{1.75f, 4.0f}, {1.75f, 4.0f}}, {{1.35f, 8.0f}, {1.35f, 8.0f}}, 1.0f},
-    {1, 128, 128, 256, true, {{0.95f, 3.5f}, {0.95f, 3.5f}}, {{1.1f, 6.0f}, {1.1f, 6.0f}}, 1.3f},
-    {2, 64, 32, 512, false, {{0.19f, 2.0f}, {0.33f, 2.0f}}, {{0.2f, 3.0f}, {0.33f, 3.0f}}, 1.7f},
-    {3, 32, 32, 512, false, {{0.131f, 1.1f}, {0.18f, 1.1f}}, {{0.115f, 2.5f}, {0.2f, 2.4f}}, 1.4f},
-    {4, 128, 64, 256, true, {{0.5f, 1.5f}, {0.5f, 1.5f}}, {{0.72f, 6.0f}, {0.72f, 6.0f}}, 1.1f},
+    {0, 256, 128, 512, true, {{1.75f, 4.0f}, {1.75f, 4.0f}}, {{1.58f, 8.0f}, {1.35f, 8.0f}}, 1.0f},
+    {1, 128, 128, 256, true, {{0.95f, 3.5f}, {0.87f, 3.5f}}, {{1.1f, 6.0f}, {1.1f, 6.0f}}, 1.3f},
+    {2, 64, 32, 512, false, {{0.2f, 2.29f}, {0.33f, 2.0f}}, {{0.2f, 3.0f}, {0.33f, 2.92f}}, 1.46f},
+    {3, 32, 32, 512, false, {{0.13f, 1.04f}, {0.18f, 1.1f}}, {{0.12f, 2.5f}, {0.2f, 2.4f}}, 1.44f},
+    {4, 128, 64, 256, true, {{0.57f, 1.5f}, {0.5f, 1.5f}}, {{0.87f, 6.45f}, {0.64f, 6.0f}}, 1.1f},
 };
 
 MmForm linear_mm_choose(const g4a_ctx* ctx, int mode, int bi, uint32_t M, uint32_t N, uint32_t K, bool tiles) {

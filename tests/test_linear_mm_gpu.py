@@ -72,7 +72,7 @@ EVERY_KERNEL = [
     ("0_b2_mode0", "linear", 2946, 1728, 1392, 2),
     ("0_b2_mode1", "geglu", 1635, 320, 1933, 2),
     ("0_b2_mode2", "gelu_cols", 2575, 320, 2382, 2),
-    ("0_b4_mode0", "linear", 1537, 1600, 2644, 4),
+    ("0_b4_mode0", "linear", 1175, 384, 4918, 4),
     ("0_b4_mode1", "geglu", 1594, 320, 2087, 4),
     ("0_b4_mode2", "gelu_cols", 3545, 320, 1752, 4),
     ("0_b8_mode0", "linear", 2598, 832, 1752, 8),
@@ -84,12 +84,12 @@ EVERY_KERNEL = [
     ("1_b4_mode0", "linear", 1822, 640, 4178, 4),
     ("1_b4_mode1", "geglu", 1251, 640, 4347, 4),
     ("1_b4_mode2", "gelu_cols", 3103, 704, 3542, 4),
-    ("2_b2_mode0", "linear", 409, 896, 610, 2),
+    ("2_b2_mode0", "linear", 607, 1088, 453, 2),
     ("2_b2_mode1", "geglu", 519, 320, 1456, 2),
-    ("2_b2_mode2", "gelu_cols", 407, 960, 621, 2),
-    ("2_b4_mode0", "linear", 398, 832, 662, 4),
+    ("2_b2_mode2", "gelu_cols", 357, 1088, 712, 2),
+    ("2_b4_mode0", "linear", 391, 1152, 617, 4),
     ("2_b4_mode1", "geglu", 555, 320, 1384, 4),
-    ("2_b4_mode2", "gelu_cols", 511, 896, 613, 4),
+    ("2_b4_mode2", "gelu_cols", 302, 1088, 870, 4),
     ("2_b8_mode0", "linear", 547, 640, 1377, 8),
     ("2_b8_mode2", "gelu_cols", 939, 640, 903, 8),
     ("3_b2_mode0", "linear", 27, 384, 17, 2),
@@ -106,7 +106,7 @@ EVERY_KERNEL = [
     ("4_b2_mode2", "gelu_cols", 2386, 320, 645, 2),
     ("4_b4_mode0", "linear", 1237, 320, 1328, 4),
     ("4_b4_mode1", "geglu", 551, 320, 1963, 4),
-    ("4_b4_mode2", "gelu_cols", 1413, 448, 1076, 4),
+    ("4_b4_mode2", "gelu_cols", 1477, 320, 1196, 4),
     ("4_b8_mode0", "linear", 1011, 320, 1079, 8),
     ("4_b8_mode1", "geglu", 389, 320, 2014, 8),
     ("4_b8_mode2", "gelu_cols", 2246, 320, 466, 8),
