@@ -110,9 +110,8 @@ struct g4a_ctx {
     hipFunction_t decode_short4[2] = {nullptr, nullptr};  // [dh512] four workgroups per split (quarters)
     hipFunction_t decode_short2x[2] = {nullptr, nullptr};  // the same two / four with a split's
     hipFunction_t decode_short4x[2] = {nullptr, nullptr};  // workgroups on one XCD
-    hipFunction_t decode_batch[2] = {nullptr, nullptr};   // [dh512] short decode over many sequences
-    hipFunction_t decode_wave_batch[2] = {nullptr, nullptr};  // [dh512] streaming decode over many sequences
-    hipFunction_t decode_wave_batch_kpos[2] = {nullptr, nullptr};  // [dh512] the same, explicit key positions
+    hipFunction_t decode_batch[2][2] = {};  // [one-row grid][dh512] short decode over many sequences (256: no row form)
+    hipFunction_t decode_wave_batch[2][2][2] = {};  // [explicit key positions][one-row grid][dh512] streaming decode
     hipFunction_t combine_batch[2] = {nullptr, nullptr};  // [dh512]
     hipFunction_t combine_rows[2] = {nullptr, nullptr};        // [dh512] combine of <= 16 splits
     hipFunction_t combine_rows_batch[2] = {nullptr, nullptr};  // [dh512]
@@ -807,12 +806,17 @@ int g4a_create_with(int device, const char* hsaco_path, const g4a_options* opts,
     if (int rc = get_fn(ctx, &ctx->decode_short2x[1], "g4a_decode_short2x_d512")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->decode_short4x[0], "g4a_decode_short4x_d256")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->decode_short4x[1], "g4a_decode_short4x_d512")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_batch[0], "g4a_decode_short_batch_d256")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_batch[1], "g4a_decode_short_batch_d512")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_wave_batch[0], "g4a_decode_wave_batch_d256")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_wave_batch[1], "g4a_decode_wave_batch_d512")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_wave_batch_kpos[0], "g4a_decode_wave_batch_kpos_d256")) return bail(rc);
-    if (int rc = get_fn(ctx, &ctx->decode_wave_batch_kpos[1], "g4a_decode_wave_batch_kpos_d512")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->decode_batch[0][0], "g4a_decode_short_batch_d256")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->decode_batch[0][1], "g4a_decode_short_batch_d512")) return bail(rc);
+    if (int rc = get_fn(ctx, &ctx->decode_batch[1][1], "g4a_decode_short_batch_row_d512")) return bail(rc);
+    for (int kp = 0; kp < 2; ++kp)
+        for (int row = 0; row < 2; ++row)
+            for (int d = 0; d < 2; ++d) {
+                char name[64];
+                snprintf(name, sizeof name, "g4a_decode_wave_batch%s%s_d%d", kp ? "_kpos" : "", row ? "_row" : "",
+                         d ? 512 : 256);
+                if (int rc = get_fn(ctx, &ctx->decode_wave_batch[kp][row][d], name)) return bail(rc);
+            }
     if (int rc = get_fn(ctx, &ctx->combine_batch[0], "g4a_combine_batch_d256")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->combine_batch[1], "g4a_combine_batch_d512")) return bail(rc);
     if (int rc = get_fn(ctx, &ctx->combine_rows[0], "g4a_combine_rows_d256")) return bail(rc);
@@ -1476,8 +1480,7 @@ int g4a_attention_decode_batch(g4a_ctx* ctx, const g4a_attn_args* args, uint32_t
         }
         // (see decode_wave_batch for the two grids)
         const bool one_row = L.wgs != L.max_split * L.count && (L.wave || d512);
-        hipFunction_t f = L.kpos ? ctx->decode_wave_batch_kpos[d512]
-                          : L.wave ? ctx->decode_wave_batch[d512] : ctx->decode_batch[d512];
+        hipFunction_t f = L.wave ? ctx->decode_wave_batch[L.kpos][one_row][d512] : ctx->decode_batch[one_row][d512];
         if (int rc = launch(ctx, f, one_row ? dim3(L.wgs, 1, bp.Hkv) : dim3(L.max_split, L.count, bp.Hkv),
                             dim3(L.wave ? 512 : 256, 1, 1), bp, "batched decode", true))
             return rc;

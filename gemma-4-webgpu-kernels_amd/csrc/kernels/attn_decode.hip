@@ -1514,7 +1514,10 @@ __device__ __forceinline__ void combine_row_stage(const float* __restrict__ part
 // count, sequences) grid theirs fell unevenly on the 8 XCDs, and one with more
 // than 32 (a CU holds one) ran them in two rounds: 16 sequences of 8192 .. 512
 // keys 59 -> 40 us. Equal counts take the (splits, sequences) grid, and so does the
-// short kernel at head_dim 256, whose workgroups share CUs: the search is 0.7 us.
+// short kernel at head_dim 256, whose workgroups share CUs: the search is 0.7 us. The
+// grids have kernels of their own: one that asks its grid which it is waits a round trip
+// for the answer before the first load of its sequence (32 sequences of 4096 keys at
+// head_dim 512 93.0 -> 94.6 us a step).
 __device__ __forceinline__ bool batch_params(const G4aBatchParams& b, uint32_t si, G4aDecodeParams& p) {
     const G4aSeqDesc& sd = b.seq[si];
     p = G4aDecodeParams{};
@@ -1542,10 +1545,11 @@ __device__ __forceinline__ bool batch_params(const G4aBatchParams& b, uint32_t s
     return p.nsplit > 0;
 }
 
-// This workgroup's sequence and split: (splits, sequences) grids give them, else
-// (one row) the search of `first` does, one entry per lane.
+// This workgroup's sequence and split, as the (splits, sequences) grid gives them or
+// (ROW) by a search of `first`, one entry per lane.
+template <bool ROW>
 __device__ __forceinline__ uint32_t batch_item(const G4aBatchParams& b, uint32_t& split) {
-    if (gridDim.y > 1) {
+    if (!ROW) {
         split = blockIdx.x;
         return blockIdx.y;
     }
@@ -1555,19 +1559,19 @@ __device__ __forceinline__ uint32_t batch_item(const G4aBatchParams& b, uint32_t
     return __builtin_amdgcn_readfirstlane(si);
 }
 
-template <int DH>
+template <int DH, bool ROW>
 __device__ __forceinline__ void decode_short_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
     uint32_t split;
-    if (!batch_params(b, batch_item(b, split), p) || split >= p.nsplit) return;
+    if (!batch_params(b, batch_item<ROW>(b, split), p) || split >= p.nsplit) return;
     decode_short<DH>(p, split, 0u);
 }
 
-template <int DH, bool KPOS>
+template <int DH, bool KPOS, bool ROW>
 __device__ __forceinline__ void decode_wave_batch(const G4aBatchParams& b) {
     G4aDecodeParams p;
     uint32_t split;
-    if (!batch_params(b, batch_item(b, split), p) || split >= p.nsplit) return;
+    if (!batch_params(b, batch_item<ROW>(b, split), p) || split >= p.nsplit) return;
     decode_wave<DH, KPOS>(p, split, 0u);
 }
 
@@ -1741,17 +1745,28 @@ __global__ __launch_bounds__(256) void g4a_decode_short4x_d256(G4aDecodeParams p
 __global__ __launch_bounds__(256) void g4a_decode_short4x_d512(G4aDecodeParams p) {
     decode_short<512, 4>(at_device_pos(p), (blockIdx.x & 7u) + 8u * (blockIdx.x >> 5), blockIdx.y, (blockIdx.x >> 3) & 3u);
 }
-__global__ __launch_bounds__(256) void g4a_decode_short_batch_d256(G4aBatchParams b) { decode_short_batch<256>(b); }
-__global__ __launch_bounds__(256) void g4a_decode_short_batch_d512(G4aBatchParams b) { decode_short_batch<512>(b); }
-__global__ __launch_bounds__(512) void g4a_decode_wave_batch_d256(G4aBatchParams b) { decode_wave_batch<256, false>(b); }
-__global__ __launch_bounds__(512) void g4a_decode_wave_batch_d512(G4aBatchParams b) { decode_wave_batch<512, false>(b); }
-// sequences with explicit key positions (every descriptor of the launch has kpos set)
-__global__ __launch_bounds__(512) void g4a_decode_wave_batch_kpos_d256(G4aBatchParams b) {
-    decode_wave_batch<256, true>(b);
+__global__ __launch_bounds__(256) void g4a_decode_short_batch_d256(G4aBatchParams b) { decode_short_batch<256, false>(b); }
+__global__ __launch_bounds__(256) void g4a_decode_short_batch_d512(G4aBatchParams b) { decode_short_batch<512, false>(b); }
+__global__ __launch_bounds__(256) void g4a_decode_short_batch_row_d512(G4aBatchParams b) {
+    decode_short_batch<512, true>(b);
 }
-__global__ __launch_bounds__(512) void g4a_decode_wave_batch_kpos_d512(G4aBatchParams b) {
-    decode_wave_batch<512, true>(b);
-}
+// _kpos: sequences with explicit key positions (every descriptor of the launch has kpos
+// set); _row: on one row of workgroups
+#define G4A_WAVE_BATCH(DH)                                                                                       \
+    __global__ __launch_bounds__(512) void g4a_decode_wave_batch_d##DH(G4aBatchParams b) {                       \
+        decode_wave_batch<DH, false, false>(b);                                                                  \
+    }                                                                                                            \
+    __global__ __launch_bounds__(512) void g4a_decode_wave_batch_row_d##DH(G4aBatchParams b) {                   \
+        decode_wave_batch<DH, false, true>(b);                                                                   \
+    }                                                                                                            \
+    __global__ __launch_bounds__(512) void g4a_decode_wave_batch_kpos_d##DH(G4aBatchParams b) {                  \
+        decode_wave_batch<DH, true, false>(b);                                                                   \
+    }                                                                                                            \
+    __global__ __launch_bounds__(512) void g4a_decode_wave_batch_kpos_row_d##DH(G4aBatchParams b) {              \
+        decode_wave_batch<DH, true, true>(b);                                                                    \
+    }
+G4A_WAVE_BATCH(256)
+G4A_WAVE_BATCH(512)
 __global__ __launch_bounds__(COMBINE_THREADS) void g4a_combine_batch_d256(G4aBatchParams b) { combine_batch<256>(b); }
 __global__ __launch_bounds__(COMBINE_THREADS) void g4a_combine_batch_d512(G4aBatchParams b) { combine_batch<512>(b); }
 __global__ __launch_bounds__(256) void g4a_combine_rows_batch_d256(G4aBatchParams b) { combine_rows_batch<256>(b); }

@@ -62,11 +62,11 @@ constexpr uint32_t G4A_BATCH_SEQ = 64;
 // Arguments of a batched decode launch: sequences seq[0 ..) and the shape they
 // share. Workgroup i of a one-row decode grid runs split i - first[s] of the last
 // sequence s with first[s] <= i (past the launch's sequences: 2^32 - 1); other
-// grids are (splits, sequences), a wide combine's (dims, heads, sequences). A sequence's partials are laid out as
-// G4aDecodeParams::part for T = 1 and its split count.
+// grids are (splits, sequences), a wide combine's (dims, heads, sequences). A
+// sequence's partials are laid out as G4aDecodeParams::part for T = 1 and its split
+// count.
 struct G4aBatchParams {
     G4aSeqDesc seq[G4A_BATCH_SEQ];
-    uint32_t first[G4A_BATCH_SEQ];
     float* part;
     const float* dummy;
     const uint32_t* kpos;  // the explicit key positions of the launch's sequences (device)
@@ -75,6 +75,7 @@ struct G4aBatchParams {
     uint32_t ring_cap;
     uint32_t window;
     float scale, softcap;
+    uint32_t first[G4A_BATCH_SEQ];
 };
 
 static_assert(sizeof(G4aBatchParams) <= 4096, "batched decode arguments fit the kernel argument segment");
