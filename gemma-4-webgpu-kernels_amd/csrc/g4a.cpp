@@ -1811,7 +1811,7 @@ LinearChoice choose_linear(const g4a_ctx* ctx, int mode, const g4a_qweight* w, c
 // busy; 8-bit weights take `wide` times as long). Against every form at 13 M = 17 ..
 // 2048 of [2048, 1536], [1536, 2048 .. 12288], [4096, 1536], [256, 1536] and gate + up
 // [6144, 1536], [12288, 1536] weights at 2, 4 and 8 bits (390 calls), the choice is within
-// 5 % of the best in 375 and within 10 % in all but 256 weight rows at 800 .. 1024 tokens
+// 5 % of the best in 378 and within 10 % in all but 256 weight rows at 800 .. 1024 tokens
 // (2 us of 14).
 struct MmForm {
     int form;
@@ -1824,7 +1824,7 @@ struct MmForm {
 };
 constexpr MmForm MM_FORMS[5] = {
     {0, 256, 128, 512, true, {{1.75f, 4.0f}, {1.75f, 4.0f}}, {{1.58f, 8.0f}, {1.35f, 8.0f}}, 1.0f},
-    {1, 128, 128, 256, true, {{0.95f, 3.5f}, {0.87f, 3.5f}}, {{1.1f, 6.0f}, {1.1f, 6.0f}}, 1.3f},
+    {1, 128, 128, 256, true, {{0.95f, 3.5f}, {0.87f, 3.5f}}, {{1.15f, 6.0f}, {1.15f, 6.0f}}, 1.3f},
     {2, 64, 32, 512, false, {{0.2f, 2.29f}, {0.33f, 2.0f}}, {{0.2f, 3.0f}, {0.33f, 2.92f}}, 1.46f},
     {3, 32, 32, 512, false, {{0.13f, 1.04f}, {0.18f, 1.1f}}, {{0.12f, 2.5f}, {0.2f, 2.4f}}, 1.44f},
     {4, 128, 64, 256, true, {{0.57f, 1.5f}, {0.5f, 1.5f}}, {{0.87f, 6.45f}, {0.64f, 6.0f}}, 1.1f},
