@@ -416,10 +416,10 @@ PrefillSplit prefill_split_at(const PrefillTiles& tiles, uint32_t NB, const Pref
 // (8 .. 18 us from T = 173 on with every count played, ahead of it, which showed in
 // a lone call).
 // Against a sweep of fixed counts (72 calls of T = 16 .. 2048 and up to 16000 earlier
-// keys, both head_dims, with and without a window) the choice is within 5 % of the best,
-// 6 % at 300 tokens and 9 % (3 us) at 64 of head_dim 512 (us, one workgroup a block ->
-// chosen): hd512 T = 173 after 6001 keys 1029 -> 159, 16 after 16000 2639 -> 123, T = 2048
-// 357 -> 297, 231 74 -> 44; hd256 window 512, T = 2048 unchanged, 512 79 -> 45, 120 after
+// keys, both head_dims, with and without a window) the choice is within 5 % of the best in
+// 70, 7 % (3 and 5 us) at head_dim 512's 64 tokens and 16 after 4000 (us, one workgroup a
+// block -> chosen): hd512 T = 173 after 6001 keys 1029 -> 159, 16 after 16000 2639 -> 123,
+// T = 2048 357 -> 297, 231 74 -> 44; hd256 window 512, T = 2048 unchanged, 512 79 -> 45, 120 after
 // 3000 83 -> 41. A few workgroups more than CUs cost a second round, which a part of one
 // left over in the play must count for: 513 after 3000 312 -> 240, 700 89 -> 72.
 constexpr uint32_t PF_SIM_CUS = 32;

@@ -249,10 +249,11 @@ __device__ __forceinline__ void copy4s_to_lds(const void* sbase, uint32_t voff, 
 // TB = 2 a wave issues 32 MFMAs (1024 cycles) per step with one operand set being read
 // and unpacked ahead of them; with the reads placed where used, a step took 1.3 us
 // instead of 0.8 (4 waves, one workgroup). Bound by the MFMAs and the vector
-// instructions between them, which do not overlap: with every CU busy the matrix pipe
-// works half the cycles, and the clock falls from 2.4 to 1.8 GHz. Gate + up 4-bit
-// [6144, 1536] at M = 2048 takes 154 us (1000 TFLOP/s of fp16 products), 235 with three
-// bf16 parts; 161 with 64-bit copy addresses per lane and the sums cleared after a fold.
+// instructions between them, which do not overlap: of the cycles with every CU busy the
+// matrix pipe works 0.53 and the other vector instructions issue in 0.40 (counters), at a
+// clock that falls from 2.4 to 1.8 GHz. Gate + up 4-bit [6144, 1536] at M = 2048 takes 152
+// us (1020 TFLOP/s of fp16 products), 235 with three bf16 parts; 7 more with 64-bit copy
+// addresses per lane and the sums cleared after a fold.
 template <int BITS, int MODE, int NW, int TB>
 __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
     constexpr int XF = 4096 * TB;                // floats of a step's x tile (2 TB token blocks)
@@ -451,9 +452,11 @@ __device__ __forceinline__ void linear_mm_tile(const G4aLinearMmParams& p) {
 // Fewer rows: workgroup = 32 RB weight rows (of each weight) x 32 TB tokens, its 8
 // waves taking every eighth 64-k step, operands straight from memory (x from L2),
 // the waves' sums added through LDS in order. The tiles above would leave most CUs
-// idle here: [1536, 6144] at M = 120 takes 24 us, 100 as 128 x 128 tiles, 91 with
-// three bf16 parts and no k split. Bound by x through L2 (8 KiB per step and token
-// block for 8 RB MFMAs).
+// idle here: [1536, 6144] at M = 120 takes 20 us, 100 as 128 x 128 tiles, 91 with
+// three bf16 parts and no k split. Bound by the round trips of a wave's few steps: at
+// [2048, 1536] M = 120 the waves wait for loads in 43 % of their cycles and to issue in
+// 38 %, vector instructions take 12 % (counters); the 59 MB that come through L2 in 6.5 us
+// are a quarter of what it gives.
 template <int BITS, int MODE, int RB, int TB>
 __device__ __forceinline__ void linear_mm_ksplit(const G4aLinearMmParams& p) {
     constexpr int NWT = MODE == 1 ? 2 : 1;  // weights
@@ -658,13 +661,15 @@ __device__ __forceinline__ constexpr int mm_few_x(int i, int pos) {
 // 16 rows of x or fewer (a serving batch's step): workgroup = 16 RB weight rows (of
 // each weight), NW waves taking every NW-th 64-k step, x split in registers by the
 // wave that uses it (a launch ahead for it would cost 3 us), one scale per token and
-// step; the waves' sums added through LDS in order. Bound by latency and by x
-// through L2: three steps' loads are in flight and none past the last step is made
-// (those loads alone were 5 of 12 us at M = 16). [2048, 1536] at M = 12 takes 5.8 us,
-// gate + up [6144, 1536] 9.8, [1536, 6144] 14.7 (7.2, 19.0 and 19.3 as words; NW = 8).
+// step; the waves' sums added through LDS in order. Bound by each wave's chain of
+// steps: at [1536, 6144] M = 12 its cycles are half waits for loads, a quarter waits to
+// issue and a quarter vector instructions (counters; L2 delivers 33 MB in 14.6 us, no
+// limit). Three steps' loads are in flight and none past the last step is made (those
+// loads alone were 5 of 12 us at M = 16). [2048, 1536] at M = 12 takes 5.8 us, gate + up
+// [6144, 1536] 9.8, [1536, 6144] 14.7 (7.2, 19.0 and 19.3 as words; NW = 8).
 // NW = 16 halves the chain of a row of 16 .. 32 steps: [2048, 1536] M = 12 5.5 -> 5.1,
-// M = 2 4.4 -> 4.0, [1536, 2048] M = 4 5.2 -> 4.8. Longer rows wait for x through L2
-// instead ([1536, 4096] M = 8 8.4 against 9.0), shorter ones have no step for each wave.
+// M = 2 4.4 -> 4.0, [1536, 2048] M = 4 5.2 -> 4.8. Longer rows lose ([1536, 4096] M = 8
+// 8.4 against 9.0), shorter ones have no step for each wave.
 template <int BITS, int MODE, int RB, int NW>
 __device__ __forceinline__ void linear_mm_few(const G4aLinearMmParams& p) {
     constexpr int NWT = MODE == 1 ? 2 : 1;

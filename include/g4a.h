@@ -59,8 +59,9 @@ typedef struct g4a_options {
     uint32_t short_max_wgs;   /* 4 (default), 2 or 1: workgroups sharing one short-kernel split */
     int32_t batch_kernel;     /* g4a_attention_decode_batch: 0 (default) automatic, 1 short, 2 streaming */
     uint32_t batch_keys_per_split; /* streaming batch launches: 0 (default) automatic */
-    int32_t linear_i8;        /* -1 (default): the int8 matrix-core projection for M <= 2 weights of
-                                 16 MB and more; 1: for every eligible weight; 0: never */
+    int32_t linear_i8;        /* -1 (default): the int8 matrix-core projection for M <= 2 and weights of
+                                 16 MB and more, M <= 8 from 64 MiB; 1: for every eligible weight at
+                                 M <= 2; 0: never */
     int32_t fuse_projection;  /* 0 (default); 1: g4a_attention_linear_q merges a decode step's
                                  split partials inside its projection (2..16 splits, short-weight
                                  projections): bit-identical, measured slower on MI355X */
@@ -143,18 +144,19 @@ int g4a_attention(g4a_ctx *ctx, const g4a_attn_args *args);
  * callers that cannot allocate while they run (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). Same arguments, same
  * kernels and the same results (bit-identical) as g4a_attention, except that a
- * call's split partials and pre-split K/V live in a static scratch array of
- * G4A_NOALLOC_SCRATCH_BYTES compiled into libg4a.so instead of the context's
- * workspace, and that it calls no allocator. Each GPU holds its own copy of the
- * array, looked up (and so loaded onto the GPU) by the first no-alloc call or
+ * call's split partials and pre-split K/V live in a static scratch array
+ * compiled into libg4a.so instead of the context's workspace, and that it calls no
+ * allocator: G4A_NOALLOC_SCRATCH_BYTES, which decide what it refuses, and 34 MiB behind
+ * them that only the partials of a prefill's split query blocks take. Each GPU holds its
+ * own copy of the array, looked up (and so loaded onto the GPU) by the first no-alloc call or
  * graph capture on that GPU, and held until the process ends: a process that
  * does neither does not hold it.
  * Fails with G4A_E_UNSUPPORTED, enqueueing nothing, when the call needs more
  * scratch than the array holds (decode: T*Hq*splits*(Dh+2)*4 bytes for more
- * than one split; prefill: about 2*keys*Hkv*Dh*4 bytes plus the partials of
- * split query blocks at head_dim 512; g4a_attention_plan gives the decode
- * figure) or passes non-contiguous explicit positions (they are staged through
- * allocated buffers). Every call on a GPU shares that GPU's array and leaves
+ * than one split; prefill: about 2*keys*Hkv*Dh*4 bytes, and at head_dim 512 two
+ * 129 KiB partials per kv head for each block of 8 queries with more keys than the
+ * average block; g4a_attention_plan gives the decode figure) or passes
+ * non-contiguous explicit positions (they are staged through allocated buffers). Every call on a GPU shares that GPU's array and leaves
  * its contents behind (nothing in it needs clearing: each call writes what it
  * reads first), so calls that overlap on one GPU race: keep them on one stream
  * or order them with events. */
@@ -408,6 +410,13 @@ int g4a_embed_rows_q(g4a_ctx *ctx, const g4a_qweight *table, const uint32_t *ids
  * (explicit position arrays, embedding ids), a larger workspace or a new RoPE
  * table, and g4a_h2d / g4a_d2h / g4a_zero / g4a_sync / the timers, fail with
  * G4A_E_ARG while a capture is open: run such calls once before capturing.
+ * Three calls that could use a larger workspace are recorded in a form that fits
+ * the one there is, slower and with another order of sums than the eager call's:
+ * a prefill in fewer workgroups per query block (16 queries after 16000 keys: up
+ * to 2.6 ms instead of 0.12), a projection of 16 and more rows on three bf16 parts,
+ * a decode batch in fewer splits. Run once eagerly before, they are recorded as the
+ * eager call runs, bit for bit. On a device without the memory for the larger
+ * workspace, eager calls take the same forms.
  * After any failing call that enqueues work inside a capture, still call
  * g4a_capture_end, which then returns that first failure's code and no graph
  * (the recording would lack the refused call); a failing query

@@ -123,3 +123,16 @@ def test_a_captured_batch_takes_the_splits_its_workspace_has_room_for(ctx):
     assert _batch(ctx, 128, 160) == got
     hip.budget()
     assert _batch(ctx, 128, 160) == 2 * [("g4a_decode_wave_batch_d512", 4), ("g4a_combine_rows_batch_d512", 8)]
+
+
+def test_a_capture_after_the_eager_call_records_its_kernels(ctx):
+    def calls():
+        got = _attend(ctx, 8192) + _project(ctx, 3000)
+        return got + _batch(ctx, 128, 160)
+
+    calls()
+    eager = calls()  # (the workspace is there by now)
+    ctx.capture_begin()
+    captured = calls()
+    ctx.capture_end().free()
+    assert captured == eager and "g4a_prefill_merge_d512" in eager and "g4a_split_x_b4" in eager
