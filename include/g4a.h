@@ -156,10 +156,11 @@ int g4a_attention(g4a_ctx *ctx, const g4a_attn_args *args);
  * than one split; prefill: about 2*keys*Hkv*Dh*4 bytes, and at head_dim 512 two
  * 129 KiB partials per kv head for each block of 8 queries with more keys than the
  * average block; g4a_attention_plan gives the decode figure) or passes
- * non-contiguous explicit positions (they are staged through allocated buffers). Every call on a GPU shares that GPU's array and leaves
- * its contents behind (nothing in it needs clearing: each call writes what it
- * reads first), so calls that overlap on one GPU race: keep them on one stream
- * or order them with events. */
+ * non-contiguous explicit positions (they are staged through allocated buffers).
+ * Every call on a GPU shares that GPU's array and leaves its contents behind
+ * (nothing in it needs clearing: each call writes what it reads first), so calls
+ * that overlap on one GPU race: keep them on one stream or order them with
+ * events. */
 #define G4A_NOALLOC_SCRATCH_BYTES (64u << 20)
 int g4a_attention_noalloc(g4a_ctx *ctx, const g4a_attn_args *args);
 
