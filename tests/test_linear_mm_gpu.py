@@ -212,12 +212,8 @@ def test_scales_apart_and_non_finite_rows(ctx, M):
     assert np.array_equal(got[5], oracle.linear_q(x[5:6], w)[0], equal_nan=True)
 
 
-@pytest.mark.parametrize("bits,signed", [(4, False), (2, False), (8, True)])
-@pytest.mark.parametrize("M", [9, 20, 400])
-def test_activations_beside_outliers_keep_their_bits(ctx, M, bits, signed):
-    # one |x| of 2^26 times the others in every 64 k, where every weight is 0: the outputs are
-    # sums of the others, held to the bound of f32 sums of those alone
-    N, K = 2048, 1024
+def _beside_outliers(power, N, K, M, bits, signed):
+    """Normal activations, one of 2^power in every 64, and weights that are 0 there."""
     qb, sc, g = synth.quant_weight(13, N, K, bits, signed_i8=signed, group_size=None)
     qb = np.array(qb, np.uint8).reshape(N, -1)
     x = synth.normal_f32(14, 1, M * K).reshape(M, K).copy()
@@ -226,13 +222,37 @@ def test_activations_beside_outliers_keep_their_bits(ctx, M, bits, signed):
         shift = bits * (k % per)
         zero = 0 if signed else (1 << (bits - 1)) << shift
         qb[:, k // per] = (qb[:, k // per] & (0xFF ^ (((1 << bits) - 1) << shift))) | zero
-        x[:, k] = np.float32(2.0 ** 26)
-    w = oracle.QWeight(qb, sc, N, K, bits, signed, g)
+        x[:, k] = np.float32(2.0 ** power)
+    return oracle.QWeight(qb, sc, N, K, bits, signed, g), x
+
+
+@pytest.mark.parametrize("bits,signed", [(4, False), (2, False), (8, True)])
+@pytest.mark.parametrize("M", [9, 20, 400])
+def test_activations_beside_outliers_keep_their_bits(ctx, M, bits, signed):
+    # one |x| of 2^26 times the others in every 64 k, where every weight is 0: the outputs are
+    # sums of the others, held to the bound of f32 sums of those alone
+    w, x = _beside_outliers(26, 2048, 1024, M, bits, signed)
     print(f"[gpu] M={M} b{bits}", flush=True)
     with Dev(ctx) as d:
-        y = d.empty((M, N))
+        y = d.empty((M, 2048))
         ctx.linear_q(d.w(w), d.arr(x).ptr, y.ptr, M)
         _check_sum(y.to_host(), oracle.linear_q(x, w), _bound(x, w), f"M={M} b{bits}")
+
+
+@pytest.mark.parametrize("M", [9, 20, 400])
+def test_activations_far_below_an_outlier_keep_2_to_the_minus_50_of_it(ctx, M):
+    # 2^36 times the others: each is held to 2^-50 of that, 2^-14, so an output misses the f32
+    # bound by at most 2^-14 * sum |w|
+    w, x = _beside_outliers(36, 2048, 1024, M, 4, False)
+    print(f"[gpu] M={M}", flush=True)
+    with Dev(ctx) as d:
+        y = d.empty((M, 2048))
+        ctx.linear_q(d.w(w), d.arr(x).ptr, y.ptr, M)
+        got = y.to_host().astype(np.float64)
+    rounding = 2.0 ** -14 * _bound(np.ones((1, 1024), np.float32), w)
+    err = np.abs(got - oracle.linear_q(x, w))
+    print(f"  worst err / bound {(err / (2e-6 * _bound(x, w) + 1e-7 + rounding)).max():.3f}", flush=True)
+    assert np.all(err <= 2e-6 * _bound(x, w) + 1e-7 + rounding)
 
 
 @pytest.mark.parametrize("M", [3, 8, 9])
