@@ -37,7 +37,7 @@ constexpr uint32_t PREFILL_MIN_T = 16;
 constexpr float PREFILL_TAU_MIN = 7.0f;
 constexpr float PREFILL_TAU_LOGN = 2.0f;
 // The prefill split's cost model (prefill_split), in the time of one 16-key tile
-// of a workgroup (1.3 us at head_dim 256, 2.6 at 512): a workgroup's fixed cost,
+// of a workgroup (about 1.4 us at head_dim 256, 2.3 at 512): a workgroup's fixed cost,
 // the merge launch, a partial slot's write and read; the fewest tiles worth a
 // share; and the most partial slots of a call (129 KiB each at head_dim 512).
 constexpr float PREFILL_WG_TILES_256 = 18.0f;
